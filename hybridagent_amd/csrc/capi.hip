@@ -80,7 +80,32 @@ struct AddNorm {
   uint16_t* y;
 };
 
+// Rows up to which the shared MLP's linears stream their weights
+// (k_linear_bf16, 64 rows per pass); above, the tiled GEMM.  FFN block (H =
+// 2816, Im = 2112) at 65 / 96 / 128 / 300 / 2048 rows: streamed 180 / 194 /
+// 244 / 331 / 1237 us, tiled 186 / 188 / 226 / 246 / 506 us.
+constexpr int64_t kLinearStreamMaxM = 80;
+
+// The BF16 experts' routed rows up to which their weights stream once per
+// 16..64 rows of an expert (k_bf16_expert); above, the tiled GEMM (an
+// expert's weights once per 128 rows).  Gemma shape at 128 / 256 / 512 / 8248
+// rows: 192 / 267 / 315 / 1341 us streamed, 178 / 243 / 271 / 329 us tiled;
+// with Zipf-skewed routing 135 / 202 / 335 us against 142 / 158 / 231.
+constexpr int64_t kBf16StreamMaxRows = 192;
+
 inline hipError_t launch_linear_call(const LinearCall& l, hipStream_t s) {
+  if ((l.epi == kLinGateUp || l.epi == kLinPlain) && l.M > kLinearStreamMaxM && gemm_bf16_supported(l.K, l.N)) {
+    GemmBf16Args a{};
+    a.act = l.x;
+    a.W = l.W;
+    a.W2 = l.W2;
+    a.out = l.out;
+    a.M = (int)l.M;
+    a.cols = l.N;
+    a.K = l.K;
+    a.mb = gemm_bf16_blocks(l.M, l.epi == kLinGateUp ? 2 * (int64_t)l.N : l.N);
+    return launch_gemm_bf16(l.epi == kLinGateUp ? kGemmGateUp : kGemmPlain, a, 0, s);
+  }
   return launch_linear_bf16(l.epi, l.x, l.W, l.W2, l.bias, l.res, l.out, l.M, l.N, l.K, s);
 }
 
@@ -987,9 +1012,42 @@ int moe_bf16_experts_forward(const uint16_t* hidden, const int64_t* topk_idx, co
   hipError_t e =
       M * top_k > kSortMultiMinRows
           ? launch_sort_multi(topk_idx, (int)M, (int)top_k, (int)E, L.sorted_pos, L.offsets, L.desc,
-                              L.counters, L.tiles, L.blockcnt, kPrefillBM, 0, s)
+                              L.counters, L.tiles, L.blockcnt, kPrefillBM, 0, s, L.queues)
           : launch_sort(topk_idx, (int)M, (int)top_k, (int)E, L.sorted_pos, L.offsets, L.desc,
-                        L.counters, L.tiles, kPrefillBM, 0, s);
+                        L.counters, L.tiles, kPrefillBM, 0, s, L.queues);
+  // the tile list holds an expert's tile index in 16 bits
+  if (M * top_k > kBf16StreamMaxRows && M * top_k <= int64_t(65535) * kPrefillBM && gemm_bf16_supported(H, I) &&
+      gemm_bf16_supported(I, H)) {
+    GemmBf16Args g{};
+    g.sorted_pos = L.sorted_pos;
+    g.offsets = L.offsets;
+    g.tiles = L.tiles;
+    g.counters = L.counters;
+    g.topk = (int)top_k;
+    g.rows_total = (int)(M * top_k);
+    g.M = (int)M;
+    g.act = hidden;
+    g.W = gate_up_proj;
+    g.W2 = gate_up_proj + I * H;
+    g.wrows = 2 * I;
+    g.out = L.inter;
+    g.cols = (int)I;
+    g.K = (int)H;
+    g.queue = L.queues;
+    const int mt = max_mtiles(M, top_k, E);
+    if (e == hipSuccess) e = launch_gemm_bf16(kGemmGateUp, g, mt, s);
+    g.act = L.inter;
+    g.W = down_proj;
+    g.W2 = nullptr;
+    g.wrows = H;
+    g.out = L.dn;
+    g.cols = (int)H;
+    g.K = (int)I;
+    g.queue = L.queues + kPrefillQueueInts / 2;
+    if (e == hipSuccess) e = launch_gemm_bf16(kGemmPlain, g, mt, s);
+    if (e == hipSuccess) e = launch_combine(L.dn, topk_idx, topk_w, out, (int)M, (int)top_k, (int)E, (int)H, s);
+    return launch_status(e);
+  }
   const int max_slots = (int)(M * top_k < E ? M * top_k : E);
   Bf16ExpertArgs a{};
   a.sorted_pos = L.sorted_pos;

@@ -58,6 +58,7 @@
 // wait counts the loads that wavefront issued after it.
 #include "common.hpp"
 #include "launch.hpp"
+#include "lds_pipe.hpp"
 
 namespace w4a16 {
 
@@ -100,43 +101,6 @@ constexpr int px_wide_b(int b) { return b == 0 ? kPxBOff : 4096 + 8192 * (b - 1)
 constexpr int px_wide_s(int b) { return b == 0 ? kPxSOff : 4096 + 8192 * (kPxWide - 1) + 4096 * (b - 1); }
 static_assert(px_wide_s(kPxWide - 1) + 4096 <= kPxBOff, "a wide stage's blocks fit in the A region");
 static_assert(kPrefillTinyRows == 32, "a wide item is one 32-row m-block");
-
-
-// s_waitcnt immediate for vmcnt <= n with expcnt and lgkmcnt not waited for
-// (gfx9 encoding: vmcnt bits 3:0 and 15:14, expcnt 6:4, lgkmcnt 11:8)
-constexpr int px_vm_wait(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8); }
-
-// s_waitcnt vmcnt(n) for a wavefront-uniform n <= 7
-__device__ __forceinline__ void px_wait_vm(int n) {
-  switch (n) {
-    case 1: __builtin_amdgcn_s_waitcnt(px_vm_wait(1)); break;
-    case 2: __builtin_amdgcn_s_waitcnt(px_vm_wait(2)); break;
-    case 3: __builtin_amdgcn_s_waitcnt(px_vm_wait(3)); break;
-    case 4: __builtin_amdgcn_s_waitcnt(px_vm_wait(4)); break;
-    case 5: __builtin_amdgcn_s_waitcnt(px_vm_wait(5)); break;
-    case 6: __builtin_amdgcn_s_waitcnt(px_vm_wait(6)); break;
-    case 7: __builtin_amdgcn_s_waitcnt(px_vm_wait(7)); break;
-    default: __builtin_amdgcn_s_waitcnt(px_vm_wait(0)); break;
-  }
-}
-
-// Workgroup barrier for LDS data only: each wavefront waits for its own LDS
-// operations, then meets the others.  (__syncthreads() would also wait for
-// every global load in flight, the direct LDS loads of the next stages
-// included.)
-__device__ __forceinline__ void px_barrier() {
-  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
-
-// direct global -> LDS load: lane l's 16 bytes land at lds_dst + 16 l
-__device__ __forceinline__ void px_dma16(__amdgpu_buffer_rsrc_t rsrc, int voff, int soff, void* lds_dst) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void*)lds_dst, 16,
-                                          voff, soff, 0, 0);
-}
-
-__device__ __forceinline__ f32x16_t mfma32x(u32x4_t a, u32x4_t b, f32x16_t c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(a), as_bf16x8(b), c, 0, 0, 0);
-}
 
 }  // namespace
 
@@ -439,7 +403,7 @@ __device__ __forceinline__ int px_run(const PrefillArgs& a, unsigned char* smem,
   // operand, the activation rows its B operand
   auto mfmas = [&](const u32x4_t* af, u32x4_t bf) {
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb) acc[mb] = mfma32x(bf, af[mb], acc[mb]);
+    for (int mb = 0; mb < MB; ++mb) acc[mb] = mfma32(bf, af[mb], acc[mb]);
   };
   auto stage_ptr = [&](int sl) -> const unsigned char* { return smem + sl * kPxStageBytes; };
   // the loads issued after the awaited stage: those of the stage issued in
@@ -488,7 +452,7 @@ __device__ __forceinline__ int px_run(const PrefillArgs& a, unsigned char* smem,
         const u32x4_t bfn = unpack_exact<false>(wv[s2 + 1], es, kr);
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb) {
-          acc[mb] = mfma32x(bf, af[mb], acc[mb]);
+          acc[mb] = mfma32(bf, af[mb], acc[mb]);
           af[mb] = *reinterpret_cast<const u32x4_t*>(st + mb * 4096 + aoff[s2 + 1]);
         }
         bf = bfn;
@@ -501,7 +465,7 @@ __device__ __forceinline__ int px_run(const PrefillArgs& a, unsigned char* smem,
         const uint32_t sp = *reinterpret_cast<const uint32_t*>(sn + soff_of(t + 1));
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb) {
-          acc[mb] = mfma32x(bf, af[mb], acc[mb]);
+          acc[mb] = mfma32(bf, af[mb], acc[mb]);
           af[mb] = *reinterpret_cast<const u32x4_t*>(sn + mb * 4096 + aoff[0]);
         }
         sc = scale_of(t + 1, sp);
@@ -664,7 +628,7 @@ __device__ __forceinline__ int px_run_w(const PrefillArgs& a, unsigned char* sme
 #pragma unroll
       for (int b = 0; b < NB; ++b) {
         const uint32_t w = s == 0 ? bw[b].x : s == 1 ? bw[b].y : s == 2 ? bw[b].z : bw[b].w;
-        acc[b] = mfma32x(unpack_exact<false>(w, es[b], kr), af, acc[b]);
+        acc[b] = mfma32(unpack_exact<false>(w, es[b], kr), af, acc[b]);
       }
     }
     wait_and_sync(n, hook);  // stage t + 1 landed (stage t + 2 may still be loading)

@@ -277,6 +277,30 @@ hipError_t launch_ffn_post(const uint16_t* mlp, const uint16_t* moe, const uint1
                            hipStream_t s);
 // BF16 experts: grid (column tile, active slot), max_slots <= 65535
 hipError_t launch_bf16_experts(int mode, Bf16ExpertArgs a, int max_slots, hipStream_t s);
+// bf16 x bf16 GEMMs at prefill sizes (kernels_gemm_bf16.hip)
+enum GemmEpilogue { kGemmGateUp = 0, kGemmPlain = 1 };
+struct GemmBf16Args {
+  const uint16_t* act;        // [M, K] rows; grouped plain: the routed rows in segment order
+  const uint16_t* W;          // plain [cols, K], gate/up the gate rows [cols, K]; grouped: the first expert's
+  const uint16_t* W2;         // gate/up: the up rows
+  uint16_t* out;              // rows of cols; grouped gate/up: routed rows, grouped plain: rows sorted_pos[s]
+  int M;                      // rows of act (grouped plain: unused)
+  int cols, K;
+  int64_t wrows;              // grouped: weight rows per expert
+  int mb;                     // dense: 32-row blocks per tile, 1 .. 5
+  // grouped (tiles non-null): the plan's 128-row tiles, its segment starts,
+  // positions and counters, the queue (9 ints, zero) and the routed rows
+  const int32_t *sorted_pos, *offsets, *tiles, *counters;
+  int32_t* queue;
+  int topk, rows_total;
+  int n_nt;                   // set by the launcher: column tiles
+};
+// K a multiple of 32 above 128, cols a multiple of 32
+bool gemm_bf16_supported(int64_t K, int64_t cols);
+// 32-row blocks per tile of a dense launch for M rows and `wrows` weight rows
+int gemm_bf16_blocks(int64_t M, int64_t wrows);
+// max_items: grouped, most m-tiles
+hipError_t launch_gemm_bf16(int epi, GemmBf16Args a, int max_items, hipStream_t s);
 // prefill grouped GEMM: one launch per stage, items = (m-tile, n-tile)
 hipError_t launch_prefill(int mode, PrefillArgs a, int max_mtiles, hipStream_t s);
 // the exact-form prefill GEMM (kernels_prefill_x.hip): H and I multiples of
