@@ -14,11 +14,21 @@
 // the chip.  Each of the eight wavefronts owns 32
 // weight rows (gate_up: 16 gate + their 16 up rows) for all the item's
 // rows: MB m-blocks of v_mfma_f32_32x32x16_bf16 accumulators (MB = 8 for
-// 256 rows; 4, 2, 1 for segment tails of up to 128, 64, 32 rows).  A tail of
-// at most 32 rows (most of them are whole experts of few rows) is a wide
-// item of three n-tiles: its stages carry three n-tiles' weights, so the
-// per-stage cost that such an item pays for little MFMA work is paid once
-// for three n-tiles, and each output is the one-n-tile item's bit for bit.
+// 256 rows; 4, 2, 1 for segment tails of up to 128, 64, 32 rows).
+//
+// The small tails (most of them are whole experts of few rows) give a stage
+// little MFMA work, so what a stage costs whatever its rows decides.
+//  - Tails of 33..64 rows, and on the packed weights of 1..32, run as tail
+//    items (px_run_t): stages of 128 k, the item's scales read once as one
+//    contiguous block.  128 experts of 64 rows at the Gemma shape, G = 128,
+//    tiled: gate_up 144 -> 116 us, down 90 -> 76 us; packed layers of 257
+//    tokens x top-8 at G = 32 / 128 322 -> 162 / 173 -> 157 us (with a 16-byte
+//    scale chunk per row and stage the 768 rows of a three-n-tile stage
+//    touched more cache lines than an XCD's L2 holds).
+//  - On the tiled weights a tail of at most 32 rows is a wide item of three
+//    n-tiles (px_run_w): one stage's cost for three n-tiles' weights.  257
+//    tokens: 140-146 us, as tail items 154 us.
+// Each output is the one-n-tile item's bit for bit.
 //
 // Per 64-wide k stage, all by direct global -> LDS loads of 16 bytes per
 // lane (one instruction fills 1 KiB).  Every load of the main loop is one,
@@ -56,6 +66,8 @@
 // order, so a vmcnt wait counted for one could pass while the other is
 // outstanding.)  Each wavefront issues only the loads it needs; a stage's
 // wait counts the loads that wavefront issued after it.
+#include <type_traits>
+
 #include "common.hpp"
 #include "launch.hpp"
 #include "lds_pipe.hpp"
@@ -83,16 +95,18 @@ constexpr int kPxTable = kPxStages * kPxStageBytes;  // 512 row indices
 constexpr int kPxEpiOff = kPxTable + 2048;
 constexpr int kPxEpiPitch = 80;
 constexpr int kPxEpiBytes = 32 * kPxEpiPitch;
-// the item index a workgroup takes from its XCD's queue (one int)
-constexpr int kPxQSlot = kPxEpiOff + kPxWaves * kPxEpiBytes;
-constexpr int kPxLds = kPxQSlot + 16;
+constexpr int kPxEpiEnd = kPxEpiOff + kPxWaves * kPxEpiBytes;
+// the item index a workgroup takes from its queue (one int), last in LDS
+constexpr int kPxLds = 160 * 1024;
+constexpr int kPxQSlot = kPxLds - 16;
+static_assert(kPxEpiEnd <= kPxQSlot, "LDS of a CU");
 // at most four direct A loads per wavefront and stage (fewer for tiles of
 // fewer rows), then one B-word load and one scale-chunk load (wavefronts
 // 0..3)
 constexpr int kPxNA = 4;
-// Wide items: a segment tail of at most kPrefillTinyRows rows (one m-block,
-// listed last by the sort) takes kPxWide n-tiles at once, so its per-stage
-// latency is paid once for three n-tiles' weights.  Its stage holds 32
+// Wide items (tiled weights): a segment tail of at most kPrefillTinyRows rows
+// (one m-block) takes kPxWide n-tiles at once, so its per-stage latency is
+// paid once for three n-tiles' weights.  Its stage holds 32
 // activation rows (4 KiB of the A region); the other n-tiles' words and
 // scale chunks go in the rest of that region: n-tile b of the item has its
 // words at px_wide_b(b) and its scale chunks at px_wide_s(b).
@@ -101,6 +115,15 @@ constexpr int px_wide_b(int b) { return b == 0 ? kPxBOff : 4096 + 8192 * (b - 1)
 constexpr int px_wide_s(int b) { return b == 0 ? kPxSOff : 4096 + 8192 * (kPxWide - 1) + 4096 * (b - 1); }
 static_assert(px_wide_s(kPxWide - 1) + 4096 <= kPxBOff, "a wide stage's blocks fit in the A region");
 static_assert(kPrefillTinyRows == 32, "a wide item is one 32-row m-block");
+// Tail items (px_run_t): a segment tail of at most 64 rows (MBT = 1 or 2
+// m-blocks).  Its stage holds 128 k: A [2 halves][32 MBT rows][128 B] | B
+// words, 16 KiB ([256 rows][64 B] from the packed layout, [2][256 rows][32 B]
+// from the tiled copy); the item's scales, whole, follow the ring of three
+// such stages (gate_up: the gate rows', the up rows' at PrefillArgs::tail_s1).
+constexpr int kPxTailMaxBlocks = 2;
+constexpr int kPxTailRing = 3;
+constexpr int px_tail_b(int mbt) { return mbt * 8192; }
+constexpr int px_tail_stage(int mbt) { return px_tail_b(mbt) + kPxBN * kPxKT; }
 
 }  // namespace
 
@@ -111,9 +134,10 @@ struct PxItem {
 };
 
 // Item `item` of a queue whose m-tiles are tile list entries x0, x0 + xs, ...:
-// m-tiles [t0, t1) of the queue (the tails of at most kPrefillTinyRows rows)
-// have n_wide items of kPxWide n-tiles each (n-tiles past the matrix compute
-// on its last rows and store nothing), the others n_nt items of one n-tile.
+// m-tiles [t0, t1) of the queue (with tiled weights the tails of at most
+// kPrefillTinyRows rows, else none) have n_wide items of kPxWide n-tiles each
+// (n-tiles past the matrix compute on its last rows and store nothing), the
+// others n_nt items of one n-tile.
 __device__ __forceinline__ PxItem px_item_info(const PrefillArgs& a, int x0, int xs, int t0, int t1, int n_wide,
                                                int item) {
   PxItem it;
@@ -143,6 +167,14 @@ __device__ __forceinline__ PxItem px_item_info(const PrefillArgs& a, int x0, int
   return it;
 }
 
+// whether a one-n-tile item runs as a tail item (px_run_t): one or two
+// m-blocks; with tiled weights two (one m-block is a wide item there)
+template <bool TILED>
+__device__ __forceinline__ bool px_is_tail(const PrefillArgs& a, const PxItem& it) {
+  if (it.mb == 2) return a.tail_s1[1] >= 0;
+  return !TILED && it.mb == 1 && a.tail_s1[0] >= 0;
+}
+
 // A lane's load sources for one item; na = the wavefront's A loads per
 // stage, n = all its loads per stage (both wavefront-uniform).
 struct PxLoads {
@@ -168,7 +200,7 @@ __device__ __forceinline__ int px_weight_row(const PrefillArgs& a, int nt, int t
 
 // gate_up reads the item's gathered rows from the LDS table, which must
 // hold this item's rows (row r at entry seg0 % 4 + r)
-template <int MODE>
+template <int MODE, bool TILED>
 __device__ __forceinline__ PxLoads px_loads(const PrefillArgs& a, const PxItem& it, const unsigned char* smem) {
   PxLoads L;
   const int lane = threadIdx.x & 63;
@@ -193,7 +225,7 @@ __device__ __forceinline__ PxLoads px_loads(const PrefillArgs& a, const PxItem& 
   // B words: instruction `wave` brings tile rows 32 wave .. + 31, lane l row
   // 32 wave + l / 2, bytes 16 (l % 2) of the stage's 32
   const int K2 = a.K >> 1;  // packed bytes per weight row
-  if (a.wt != nullptr) {
+  if (TILED) {
     // tiled copy: the item's stage kt is the 8 KiB block (nt, kt) of the
     // expert, tile rows in order, so instruction `wave` reads one KiB
     const int nkt = a.K / kPxKT;
@@ -258,7 +290,7 @@ __device__ __forceinline__ void px_issue_table(const PrefillArgs& a, unsigned ch
 // its 32 tile rows of each n-tile, wavefronts 0..3 the scale chunks of each.
 struct PxLoadsW {
   __amdgpu_buffer_rsrc_t wsrc, ssrc;
-  int avoff, bstride;
+  int avoff;
   int bvoff[kPxWide], svoff[kPxWide];
   int na, n;
 };
@@ -277,24 +309,13 @@ __device__ __forceinline__ PxLoadsW px_loads_w(const PrefillArgs& a, const PxIte
   L.avoff = areal ? (int)(src * a.lda * 2) + 16 * chunk : 0;
   L.na = areal ? 1 : 0;
   L.n = L.na + kPxWide + (wave < 4 ? kPxWide : 0);
-  const int K2 = a.K >> 1;
-  if (a.wt != nullptr) {
-    // tiled copy: n-tiles past the expert's read past the descriptor's range
-    // (zeros); their results are not stored
-    const int nkt = a.K / kPxKT;
-    const int64_t per_e = (int64_t)a.n_nt * nkt * 2048;
-    L.wsrc = make_rsrc(reinterpret_cast<const uint32_t*>(a.wt) + (int64_t)it.e * per_e, (uint32_t)(per_e * 4));
+  // tiled copy: n-tiles past the expert's read past the descriptor's range
+  // (zeros); their results are not stored
+  const int nkt = a.K / kPxKT;
+  const int64_t per_e = (int64_t)a.n_nt * nkt * 2048;
+  L.wsrc = make_rsrc(reinterpret_cast<const uint32_t*>(a.wt) + (int64_t)it.e * per_e, (uint32_t)(per_e * 4));
 #pragma unroll
-    for (int b = 0; b < kPxWide; ++b) L.bvoff[b] = (it.nt + b) * nkt * 8192 + wave * 1024 + 16 * lane;
-    L.bstride = 8192;
-  } else {
-    L.wsrc = make_rsrc(reinterpret_cast<const uint32_t*>(a.wp) + (int64_t)it.e * a.N * (a.K >> 3),
-                       (uint32_t)a.N * K2);
-#pragma unroll
-    for (int b = 0; b < kPxWide; ++b)
-      L.bvoff[b] = px_weight_row<MODE>(a, it.nt + b, 32 * wave + (lane >> 1)) * K2 + 16 * (lane & 1);
-    L.bstride = kPxKT / 2;
-  }
+  for (int b = 0; b < kPxWide; ++b) L.bvoff[b] = (it.nt + b) * nkt * 8192 + wave * 1024 + 16 * lane;
   const uintptr_t sbase = reinterpret_cast<uintptr_t>(a.ws + (int64_t)it.e * a.N * a.ng);
   L.ssrc = make_rsrc(reinterpret_cast<const void*>(sbase & ~uintptr_t(15)), (uint32_t)a.N * a.ng * 2u + 16u);
 #pragma unroll
@@ -313,7 +334,7 @@ __device__ __forceinline__ void px_issue_w(const PrefillArgs& a, const PxLoadsW&
   unsigned char* st = smem + slot * kPxStageBytes;
   if (part == 0 && L.na > 0)
     px_dma16(make_rsrc(a.act, (uint32_t)a.act_bytes), L.avoff, kt * (kPxKT * 2), st + wave * 1024);
-  if (part < kPxWide) px_dma16(L.wsrc, L.bvoff[part < kPxWide ? part : 0], kt * L.bstride, st + px_wide_b(part) + wave * 1024);
+  if (part < kPxWide) px_dma16(L.wsrc, L.bvoff[part < kPxWide ? part : 0], kt * 8192, st + px_wide_b(part) + wave * 1024);
   if (part >= 1 && part <= kPxWide && wave < 4) {
     const int b = part >= 1 ? part - 1 : 0;
     const int gpair = ((kt * kPxKT) >> a.gshift) & ~1;
@@ -321,27 +342,201 @@ __device__ __forceinline__ void px_issue_w(const PrefillArgs& a, const PxLoadsW&
   }
 }
 
-// Issues an item's stages 0 and 1 into ring slots q0 and q0 + 1; returns the
-// wavefront's loads per stage.  Gate_up: the LDS table holds the item's rows.
+// A tail item's load sources (MBT m-blocks): MBT A loads and two B loads per
+// wavefront and stage of 128 k.
+struct PxLoadsT {
+  __amdgpu_buffer_rsrc_t asrc, wsrc;
+  int avoff, bvoff[2];
+  int bback[2];          // from a B piece past the row to the one before it
+  int bstage, bw0, bw1;  // B: bytes per stage; LDS place of load i: wave bw0 + i bw1
+};
+
+// columns of a group of 32 weight rows lie inside the matrix
 template <int MODE>
-__device__ __forceinline__ int px_issue_first(const PrefillArgs& a, const PxItem& it, unsigned char* smem, int q0) {
-  const int q1 = q0 == kPxStages - 1 ? 0 : q0 + 1;
-  if (it.nb > 1) {
+__device__ __forceinline__ bool px_group_real(const PrefillArgs& a, int nt, int g) {
+  return MODE == kModeGateUp ? 128 * nt + 16 * g < a.I : kPxBN * nt + 32 * g < a.N;
+}
+
+template <int MODE, bool TILED, int MBT>
+__device__ __forceinline__ PxLoadsT px_loads_t(const PrefillArgs& a, const PxItem& it, const unsigned char* smem) {
+  PxLoadsT L;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int* table = reinterpret_cast<const int*>(smem + kPxTable);
+  // A: instructions of 8 rows of one 64-wide half; MBT = 1: wavefront w
+  // brings rows 8 (w % 4) .. of half w / 4, MBT = 2: rows 8 w .. of both
+  const int r = 8 * (MBT == 1 ? wave & 3 : wave) + (lane >> 3);
+  const int rr = min(r, it.nrows - 1);
+  const int64_t src = MODE == kModeGateUp ? table[(it.seg0 & 3) + rr] / a.topk : it.seg0 + rr;
+  L.avoff = (int)(src * a.lda * 2) + 16 * ((lane & 7) ^ ((r >> 1) & 7));
+  L.asrc = make_rsrc(a.act, (uint32_t)a.act_bytes);
+  const int K2 = a.K >> 1;
+  if (TILED) {
+    // load i: the wavefront's KiB of k block 2 st + i
+    const int nkt = a.K / kPxKT;
+    const int64_t per_e = (int64_t)a.n_nt * nkt * 2048;
+    L.wsrc = make_rsrc(reinterpret_cast<const uint32_t*>(a.wt) + (int64_t)it.e * per_e, (uint32_t)(per_e * 4));
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      L.bvoff[i] = (it.nt * nkt + i) * 8192 + wave * 1024 + 16 * lane;
+      L.bback[i] = i * 8192;
+    }
+    L.bstage = 16384;
+    L.bw0 = 1024;
+    L.bw1 = 8192;
+  } else {
+    // load i: rows 32 wave + 16 i .., 64 bytes (four 16-byte pieces) each,
+    // piece XOR-swizzled by (row / 4) % 4
+    L.wsrc = make_rsrc(reinterpret_cast<const uint32_t*>(a.wp) + (int64_t)it.e * a.N * (a.K >> 3),
+                       (uint32_t)a.N * K2);
+    const int piece = (lane & 3) ^ ((lane >> 4) & 3);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      L.bvoff[i] = px_weight_row<MODE>(a, it.nt, 32 * wave + 16 * i + (lane >> 2)) * K2 + 16 * piece;
+      L.bback[i] = piece >= 2 ? 32 : 0;
+    }
+    L.bstage = kPxKT;
+    L.bw0 = 2048;
+    L.bw1 = 1024;
+  }
+  return L;
+}
+
+// The loads of a tail item's stage st (k blocks 2 st and 2 st + 1 of 64) into
+// ring slot `slot`.  When K / 64 is odd the last stage has only the first of
+// the two: what would come from past the row comes from the first again.
+template <int MBT>
+__device__ __forceinline__ void px_issue_t(const PrefillArgs& a, const PxLoadsT& L, unsigned char* smem, int st,
+                                           int slot) {
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  unsigned char* dst = smem + slot * px_tail_stage(MBT);
+  const int two = 2 * st + 1 < a.K / kPxKT ? 1 : 0;
+  if (MBT == 1) {
+    const int hf = wave >> 2;
+    px_dma16(L.asrc, L.avoff, (2 * st + hf * two) * (kPxKT * 2), dst + hf * 4096 + (wave & 3) * 1024);
+  } else {
+#pragma unroll
+    for (int hf = 0; hf < 2; ++hf)
+      px_dma16(L.asrc, L.avoff, (2 * st + hf * two) * (kPxKT * 2), dst + hf * 8192 + wave * 1024);
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+    px_dma16(L.wsrc, L.bvoff[i] - (two ? 0 : L.bback[i]), st * L.bstage,
+             dst + px_tail_b(MBT) + wave * L.bw0 + i * L.bw1);
+}
+
+// One contiguous block of scales (rows row0 .. of expert e) into LDS at dst,
+// from the 16-byte boundary at or before it.
+__device__ __forceinline__ void px_issue_scale_block(const PrefillArgs& a, int e, int row0, int rows,
+                                                     unsigned char* dst) {
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uintptr_t p = reinterpret_cast<uintptr_t>(a.ws + ((int64_t)e * a.N + row0) * a.ng);
+  const int bytes = (int)(p & 15) + rows * a.ng * 2;
+  const __amdgpu_buffer_rsrc_t src = make_rsrc(reinterpret_cast<const void*>(p & ~uintptr_t(15)), (uint32_t)(bytes + 15) & ~15u);
+  for (int i = wave; i * 1024 < bytes; i += kPxWaves) px_dma16(src, i * 1024 + 16 * lane, 0, dst + i * 1024);
+}
+
+// Issues a tail item's scales and its stages 0 and 1; returns the wavefront's
+// loads per stage.
+template <int MODE, bool TILED, int MBT>
+__device__ __forceinline__ int px_issue_first_t(const PrefillArgs& a, const PxItem& it, unsigned char* smem) {
+  const PxLoadsT L = px_loads_t<MODE, TILED, MBT>(a, it, smem);
+  unsigned char* s0 = smem + kPxTailRing * px_tail_stage(MBT);
+  if (MODE == kModeGateUp) {
+    const int cols = min(128, a.I - 128 * it.nt);
+    px_issue_scale_block(a, it.e, 128 * it.nt, cols, s0);
+    px_issue_scale_block(a, it.e, a.I + 128 * it.nt, cols, smem + a.tail_s1[MBT - 1]);
+  } else {
+    px_issue_scale_block(a, it.e, kPxBN * it.nt, min(kPxBN, a.N - kPxBN * it.nt), s0);
+  }
+  px_issue_t<MBT>(a, L, smem, 0, 0);
+  px_issue_t<MBT>(a, L, smem, 1, 1);
+  return MBT + 2;
+}
+
+// Issues an item's stages 0 and 1 (into the first two ring slots); returns
+// the wavefront's loads per stage.  Gate_up: the LDS table holds the item's
+// rows.  Every wavefront is past its last LDS read of the item before.
+template <int MODE, bool TILED>
+__device__ __forceinline__ int px_issue_first(const PrefillArgs& a, const PxItem& it, unsigned char* smem) {
+  if (TILED && it.nb > 1) {
     const PxLoadsW L = px_loads_w<MODE>(a, it, smem);
 #pragma unroll
-    for (int p = 0; p < 4; ++p) px_issue_w(a, L, smem, 0, q0, p);
+    for (int p = 0; p < 4; ++p) px_issue_w(a, L, smem, 0, 0, p);
 #pragma unroll
-    for (int p = 0; p < 4; ++p) px_issue_w(a, L, smem, 1, q1, p);
+    for (int p = 0; p < 4; ++p) px_issue_w(a, L, smem, 1, 1, p);
     return L.n;
   }
-  const PxLoads L = px_loads<MODE>(a, it, smem);
-  px_issue_all(a, L, smem, 0, q0);
-  px_issue_all(a, L, smem, 1, q1);
+  if (px_is_tail<TILED>(a, it)) {
+    if (!TILED && it.mb == 1) return px_issue_first_t<MODE, TILED, 1>(a, it, smem);
+    return px_issue_first_t<MODE, TILED, 2>(a, it, smem);
+  }
+  const PxLoads L = px_loads<MODE, TILED>(a, it, smem);
+  px_issue_all(a, L, smem, 0, 0);
+  px_issue_all(a, L, smem, 1, 1);
   return L.n;
 }
 
-// Multiply one item.  On entry its stages 0 and 1 are issued into slots p0
-// and p0 + 1 (this wavefront's n_inflight loads each; gate_up: the LDS table
+// The output of one group of 32 weight rows (wg) of an item for MB m-blocks
+// from block mo on.  Lane l holds, for activation row 32 mb + c of block mb,
+// the group's weight rows 8 J + 4 h + i in acc[mb][4 J + i] (J, i = 0..3):
+// four consecutive output columns per J.  gate_up stores them as 8 bytes from
+// registers: weight rows 0..15 are the gate rows and 16..31 their up rows, so
+// acc[mb][q] (gate) pairs with acc[mb][q + 8] (up).
+template <int MODE, int MB>
+__device__ __forceinline__ void px_store(const PrefillArgs& a, unsigned char* smem, const PxItem& it, int wg, int mo,
+                                         const f32x16_t* acc) {
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int h = lane >> 5, c = lane & 31;
+  if (MODE == kModeGateUp) {
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) {
+      const int grow = 32 * (mo + mb) + c;
+      if (grow >= it.nrows) continue;
+      uint16_t* orow = a.out + (int64_t)(it.seg0 + grow) * a.ldo + 128 * it.nt + 16 * wg + 4 * h;
+#pragma unroll
+      for (int J = 0; J < 2; ++J) {
+        float hv[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float g = round_bf16(acc[mb][4 * J + i]);
+          const float u = round_bf16(acc[mb][4 * J + i + 8]);
+          hv[i] = round_bf16(gelu_tanh_f32(g)) * u;
+        }
+        *reinterpret_cast<uint2*>(orow + 8 * J) = make_uint2(pack_bf16x2(hv[0], hv[1]), pack_bf16x2(hv[2], hv[3]));
+      }
+    }
+  } else {
+    // dn rows are long (N columns, rows scattered by sorted_pos): the
+    // group's 32 columns of each row go out as 16-byte stores, through LDS
+    // one m-block at a time (the wavefront reads only what it wrote: no
+    // barrier)
+    const int* table = reinterpret_cast<const int*>(smem + kPxTable);
+    unsigned char* ob = smem + kPxEpiOff + wave * kPxEpiBytes;
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) {
+#pragma unroll
+      for (int J = 0; J < 4; ++J)
+        *reinterpret_cast<uint2*>(ob + c * kPxEpiPitch + 2 * (8 * J + 4 * h)) =
+            make_uint2(pack_bf16x2(acc[mb][4 * J], acc[mb][4 * J + 1]), pack_bf16x2(acc[mb][4 * J + 2], acc[mb][4 * J + 3]));
+#pragma unroll
+      for (int itr = 0; itr < 2; ++itr) {
+        const int idx = lane + 64 * itr;
+        const int row = idx >> 2, q4 = idx & 3;
+        const int grow = 32 * (mo + mb) + row;
+        if (grow < it.nrows) {
+          const u32x4_t v = *reinterpret_cast<const u32x4_t*>(ob + row * kPxEpiPitch + 16 * q4);
+          st16(a.out + (int64_t)table[(it.seg0 & 3) + grow] * a.N + kPxBN * it.nt + 32 * wg + 8 * q4, v);
+        }
+      }
+    }
+  }
+}
+
+// Multiply one item.  On entry its stages 0 and 1 are issued into slots 0
+// and 1 (this wavefront's n_inflight loads each; gate_up: the LDS table
 // holds the item's rows).  After its last stage it issues the next item's
 // stages 0 and 1 (when has_next) and returns their per-stage load count;
 // the epilogue runs while they land.
@@ -352,9 +547,9 @@ __device__ __forceinline__ int px_issue_first(const PrefillArgs& a, const PxItem
 // With fetch_q (non-null) wavefront 0 takes an index from that queue
 // counter during the last stage (no stage load is issued after it, so the
 // stage's vmcnt(0) wait covers it) and leaves it in LDS at kPxQSlot.
-template <int MODE, int MB, bool SPLIT = false>
+template <int MODE, bool TILED, int MB, bool SPLIT = false>
 __device__ __forceinline__ int px_run(const PrefillArgs& a, unsigned char* smem, const PxItem& it,
-                                      const PxItem& nx, bool has_next, int p0, int n_inflight,
+                                      const PxItem& nx, bool has_next, int n_inflight,
                                       int* fetch_q) {
   static_assert(!SPLIT || MODE == kModeGateUp, "only gate_up has half n-tiles");
   const int lane = threadIdx.x & 63;
@@ -365,7 +560,7 @@ __device__ __forceinline__ int px_run(const PrefillArgs& a, unsigned char* smem,
   const int h = lane >> 5;  // which half of the step's 16 k this lane holds
   const int c = lane & 31;  // row (A) / column (B) inside a 32-block
   const int gshift = a.gshift;
-  const int nt = it.nt, seg0 = it.seg0, nrows = it.nrows;
+  const int nt = it.nt, seg0 = it.seg0;
 
   // this lane's reads: A fragment of block mb, step s -> row 32 mb + c,
   // chunk 4 h + s at slot chunk ^ ((c / 2) % 8); B words and scale pair of
@@ -431,12 +626,12 @@ __device__ __forceinline__ int px_run(const PrefillArgs& a, unsigned char* smem,
   float sc = 0.f;
   const ExactRegs kr = exact_regs();
   if (work) {
-    read_a(stage_ptr(p0), 0, af);
-    bw = *reinterpret_cast<const u32x4_t*>(stage_ptr(p0) + boff);
-    sc = scale_of(0, *reinterpret_cast<const uint32_t*>(stage_ptr(p0) + soff_of(0)));
+    read_a(stage_ptr(0), 0, af);
+    bw = *reinterpret_cast<const u32x4_t*>(stage_ptr(0) + boff);
+    sc = scale_of(0, *reinterpret_cast<const uint32_t*>(stage_ptr(0) + soff_of(0)));
   }
-  int slot = p0;
-  int slot2 = p0 + 2 >= kPxStages ? p0 + 2 - kPxStages : p0 + 2;
+  int slot = 0;
+  int slot2 = 2;
   // one k stage: refill the slot stage t - 1 used (issue(slot2)), multiply
   // stage t, wait for stage t + 1 and meet the other wavefronts
   auto iter = [&](int t, int n, auto issue, auto hook) {
@@ -481,7 +676,7 @@ __device__ __forceinline__ int px_run(const PrefillArgs& a, unsigned char* smem,
     slot2 = slot2 == kPxStages - 1 ? 0 : slot2 + 1;
   };
   {
-    const PxLoads lc = px_loads<MODE>(a, it, smem);
+    const PxLoads lc = px_loads<MODE, TILED>(a, it, smem);
     for (int t = 0; t + 2 < nkt; ++t)
       iter(t, lc.n, [&](int sl, int p) { px_issue(a, lc, smem, t + 2, sl, p); }, no_hook);
   }
@@ -501,69 +696,19 @@ __device__ __forceinline__ int px_run(const PrefillArgs& a, unsigned char* smem,
        [&] {
          if (fetch && lane == 0) *reinterpret_cast<int*>(smem + kPxQSlot) = fv;
        });
-  // every wavefront is past the last barrier: the next item's first two
-  // stages go into the slots of this item's stages nkt - 3 and nkt - 2
-  const int n_next = has_next ? px_issue_first<MODE>(a, nx, smem, (p0 + nkt) % kPxStages) : 0;
-  if (!work) return n_next;
-
-  // ---- epilogue.  Lane l holds, for activation row 32 mb + c of block mb,
-  // the wavefront's weight rows 8 J + 4 h + i in acc[mb][4 J + i] (J, i =
-  // 0..3): four consecutive output columns per J.  gate_up stores them as 8
-  // bytes from registers: weight rows 0..15 are the gate rows and 16..31
-  // their up rows, so acc[mb][q] (gate) pairs with acc[mb][q + 8] (up).
-#pragma unroll
-  for (int mb = 0; mb < MB && MODE == kModeGateUp; ++mb) {
-    const int grow = 32 * (mo + mb) + c;
-    if (grow >= nrows) continue;
-    {
-      uint16_t* orow = a.out + (int64_t)(seg0 + grow) * a.ldo + 128 * nt + 16 * wg + 4 * h;
-#pragma unroll
-      for (int J = 0; J < 2; ++J) {
-        float hv[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float g = round_bf16(acc[mb][4 * J + i]);
-          const float u = round_bf16(acc[mb][4 * J + i + 8]);
-          hv[i] = round_bf16(gelu_tanh_f32(g)) * u;
-        }
-        *reinterpret_cast<uint2*>(orow + 8 * J) = make_uint2(pack_bf16x2(hv[0], hv[1]), pack_bf16x2(hv[2], hv[3]));
-      }
-    }
-  }
-  if (MODE == kModeDown) {
-    // dn rows are long (N columns, rows scattered by sorted_pos): the
-    // wavefront's 32 columns of each row go out as 16-byte stores, through
-    // LDS one m-block at a time (it reads only what it wrote: no barrier)
-    const int* table = reinterpret_cast<const int*>(smem + kPxTable);
-    unsigned char* ob = smem + kPxEpiOff + wave * kPxEpiBytes;
-#pragma unroll
-    for (int mb = 0; mb < MB; ++mb) {
-#pragma unroll
-      for (int J = 0; J < 4; ++J)
-        *reinterpret_cast<uint2*>(ob + c * kPxEpiPitch + 2 * (8 * J + 4 * h)) =
-            make_uint2(pack_bf16x2(acc[mb][4 * J], acc[mb][4 * J + 1]), pack_bf16x2(acc[mb][4 * J + 2], acc[mb][4 * J + 3]));
-#pragma unroll
-      for (int itr = 0; itr < 2; ++itr) {
-        const int idx = lane + 64 * itr;
-        const int row = idx >> 2, q4 = idx & 3;
-        const int grow = 32 * mb + row;
-        if (grow < nrows) {
-          const u32x4_t v = *reinterpret_cast<const u32x4_t*>(ob + row * kPxEpiPitch + 16 * q4);
-          st16(a.out + (int64_t)table[(seg0 & 3) + grow] * a.N + kPxBN * nt + 32 * wave + 8 * q4, v);
-        }
-      }
-    }
-  }
+  // every wavefront is past its last LDS read: the next item's first stages
+  const int n_next = has_next ? px_issue_first<MODE, TILED>(a, nx, smem) : 0;
+  if (work) px_store<MODE, MB>(a, smem, it, wg, mo, acc);
   return n_next;
 }
 
 // Multiply one wide item (kPxWide n-tiles of a tail of at most 32 rows), in
-// px_run's stage protocol.  Each n-tile's outputs are px_run<MODE, 1>'s for
+// px_run's stage protocol.  Each n-tile's outputs are px_run<MODE, TILED, 1>'s for
 // that n-tile bit for bit: the same MFMA on the same operands, one k step
 // after the other.
-template <int MODE>
+template <int MODE, bool TILED>
 __device__ __forceinline__ int px_run_w(const PrefillArgs& a, unsigned char* smem, const PxItem& it,
-                                        const PxItem& nx, bool has_next, int p0, int n_inflight,
+                                        const PxItem& nx, bool has_next, int n_inflight,
                                         int* fetch_q) {
   constexpr int NB = kPxWide;
   const int lane = threadIdx.x & 63;
@@ -572,7 +717,7 @@ __device__ __forceinline__ int px_run_w(const PrefillArgs& a, unsigned char* sme
   const int h = lane >> 5;
   const int c = lane & 31;
   const int gshift = a.gshift;
-  const int nt0 = it.nt, seg0 = it.seg0, nrows = it.nrows;
+  const int nt0 = it.nt, seg0 = it.seg0;
 
   int aoff[4];
 #pragma unroll
@@ -607,8 +752,8 @@ __device__ __forceinline__ int px_run_w(const PrefillArgs& a, unsigned char* sme
   const ExactRegs kr = exact_regs();
 
   wait_and_sync(n_inflight, no_hook);  // stage 0 landed
-  int slot = p0;
-  int slot2 = p0 + 2 >= kPxStages ? p0 + 2 - kPxStages : p0 + 2;
+  int slot = 0;
+  int slot2 = 2;
   // one k stage: read its words and scales, refill the slot stage t - 1 used
   // (issue(slot2)) while multiplying, wait for stage t + 1 and meet
   auto iter = [&](int t, int n, auto issue, auto hook) {
@@ -653,66 +798,182 @@ __device__ __forceinline__ int px_run_w(const PrefillArgs& a, unsigned char* sme
        [&] {
          if (fetch && lane == 0) *reinterpret_cast<int*>(smem + kPxQSlot) = fv;
        });
-  const int n_next = has_next ? px_issue_first<MODE>(a, nx, smem, (p0 + nkt) % kPxStages) : 0;
+  const int n_next = has_next ? px_issue_first<MODE, TILED>(a, nx, smem) : 0;
 
-  // epilogue per n-tile, as px_run's for m-block 0 (n-tiles past the
-  // matrix, and gate_up columns past I, store nothing)
+  // n-tiles past the matrix, and gate_up columns past I, store nothing
 #pragma unroll
   for (int b = 0; b < NB; ++b) {
-    const int nt = nt0 + b;
-    if (MODE == kModeGateUp) {
-      if (128 * nt + 16 * wave < a.I && c < nrows) {
-        uint16_t* orow = a.out + (int64_t)(seg0 + c) * a.ldo + 128 * nt + 16 * wave + 4 * h;
-#pragma unroll
-        for (int J = 0; J < 2; ++J) {
-          float hv[4];
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const float g = round_bf16(acc[b][4 * J + i]);
-            const float u = round_bf16(acc[b][4 * J + i + 8]);
-            hv[i] = round_bf16(gelu_tanh_f32(g)) * u;
-          }
-          *reinterpret_cast<uint2*>(orow + 8 * J) = make_uint2(pack_bf16x2(hv[0], hv[1]), pack_bf16x2(hv[2], hv[3]));
-        }
-      }
-    } else if (kPxBN * nt + 32 * wave < a.N) {
-      const int* table = reinterpret_cast<const int*>(smem + kPxTable);
-      unsigned char* ob = smem + kPxEpiOff + wave * kPxEpiBytes;
-#pragma unroll
-      for (int J = 0; J < 4; ++J)
-        *reinterpret_cast<uint2*>(ob + c * kPxEpiPitch + 2 * (8 * J + 4 * h)) =
-            make_uint2(pack_bf16x2(acc[b][4 * J], acc[b][4 * J + 1]), pack_bf16x2(acc[b][4 * J + 2], acc[b][4 * J + 3]));
-#pragma unroll
-      for (int itr = 0; itr < 2; ++itr) {
-        const int idx = lane + 64 * itr;
-        const int row = idx >> 2, q4 = idx & 3;
-        if (row < nrows) {
-          const u32x4_t v = *reinterpret_cast<const u32x4_t*>(ob + row * kPxEpiPitch + 16 * q4);
-          st16(a.out + (int64_t)table[(seg0 & 3) + row] * a.N + kPxBN * nt + 32 * wave + 8 * q4, v);
-        }
-      }
-    }
+    PxItem one = it;
+    one.nt = nt0 + b;
+    if (px_group_real<MODE>(a, one.nt, wave)) px_store<MODE, 1>(a, smem, one, wave, 0, &acc[b]);
   }
   return n_next;
 }
 
-template <int MODE>
+// Multiply one tail item of MBT = MB WM m-blocks (WM = 2: gate_up's last
+// n-tile when I % 128 == 64, its four groups shared by the two wavefront
+// halves, a row block each), in px_run's protocol with stages of 128 k.  Few
+// rows give the matrix cores little work per weight, so what counts is that
+// the weights' stream and the dequantisation seldom wait: the item's scales
+// are read once, as one contiguous block (a stage's own 16-byte chunks would
+// touch a cache line per weight row and stage), and a stage takes 64
+// consecutive bytes of each packed row.  Each output is the sum px_run forms,
+// in the same order, bit for bit.
+template <int MODE, bool TILED, int MB, int WM = 1>
+__device__ __forceinline__ int px_run_t(const PrefillArgs& a, unsigned char* smem, const PxItem& it,
+                                        const PxItem& nx, bool has_next, int* fetch_q) {
+  constexpr int MBT = MB * WM;
+  constexpr int n = MBT + 2;  // loads per stage
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wg = WM == 2 ? (wave & 3) : wave;
+  const int mo = WM == 2 ? (wave >> 2) * MB : 0;
+  const int h = lane >> 5, c = lane & 31;
+  const int nkt = a.K / kPxKT, nst = (nkt + 1) >> 1;
+  const bool work = px_group_real<MODE>(a, it.nt, wg);
+  const PxLoadsT lc = px_loads_t<MODE, TILED, MBT>(a, it, smem);
+
+  // step s (0..7) of a stage: half s / 4, chunk 4 h + s % 4 of row c
+  int aoff[4];
+#pragma unroll
+  for (int s = 0; s < 4; ++s) aoff[s] = mo * 4096 + c * 128 + 16 * ((4 * h + s) ^ ((c >> 1) & 7));
+  int boff[2];
+#pragma unroll
+  for (int hf = 0; hf < 2; ++hf)
+    boff[hf] = px_tail_b(MBT) + (TILED ? hf * 8192 + (32 * wg + c) * 32 + 16 * h
+                                                 : (32 * wg + c) * 64 + 16 * ((2 * hf + h) ^ ((c >> 2) & 3)));
+  // this lane's row of scales
+  const int row0 = MODE == kModeGateUp ? (c < 16 ? 0 : a.I) + 128 * it.nt : kPxBN * it.nt;
+  const unsigned char* srow =
+      smem + (int)(reinterpret_cast<uintptr_t>(a.ws + ((int64_t)it.e * a.N + row0) * a.ng) & 15) +
+      (px_weight_row<MODE>(a, it.nt, 32 * wg + c) - row0) * a.ng * 2 +
+      (MODE == kModeGateUp && c >= 16 ? a.tail_s1[MBT - 1] : kPxTailRing * px_tail_stage(MBT));
+
+  f32x16_t acc[MB];
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int q = 0; q < 16; ++q) acc[i][q] = 0.f;
+  const ExactRegs kr = exact_regs();
+  u32x4_t af[MB], bw[2], bf;
+  float sc[2];
+  auto read_a = [&](const unsigned char* p, int s, int mb) {
+    return *reinterpret_cast<const u32x4_t*>(p + (s >> 2) * MBT * 4096 + mb * 4096 + aoff[s & 3]);
+  };
+  // a stage's words and scales (past K: the last group's, not used)
+  auto read_b = [&](const unsigned char* p, int st) {
+#pragma unroll
+    for (int hf = 0; hf < 2; ++hf) {
+      bw[hf] = *reinterpret_cast<const u32x4_t*>(p + boff[hf]);
+      const int g = min(((2 * st + hf) * kPxKT + 32 * h) >> a.gshift, a.ng - 1);
+      sc[hf] = bf16_bits_to_f32(*reinterpret_cast<const uint16_t*>(srow + 2 * g));
+    }
+  };
+  auto word = [&](int s) {
+    const u32x4_t v = bw[s >> 2];
+    return (s & 3) == 0 ? v.x : (s & 3) == 1 ? v.y : (s & 3) == 2 ? v.z : v.w;
+  };
+  auto stage_ptr = [&](int sl) -> const unsigned char* { return smem + sl * px_tail_stage(MBT); };
+  int slot = 0, slot2 = 2;
+  // one stage of NS steps: issue() fills slot2, the wait leaves VM loads in
+  // flight
+  auto stage = [&](int t, auto ns, auto vm, auto issue, auto hook) {
+    constexpr int NS = decltype(ns)::value;
+    const int nslot = slot == kPxTailRing - 1 ? 0 : slot + 1;
+    issue(slot2);
+    if (work) {
+      const unsigned char* p = stage_ptr(slot);
+#pragma unroll
+      for (int s = 0; s < NS - 1; ++s) {
+        const u32x4_t bn = unpack_exact<false>(word(s + 1), exact_scale(sc[(s + 1) >> 2]), kr);
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) {
+          acc[mb] = mfma32(bf, af[mb], acc[mb]);
+          af[mb] = read_a(p, s + 1, mb);
+        }
+        bf = bn;
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(px_vm_wait(decltype(vm)::value));
+    hook();
+    px_barrier();
+    if (work) {
+      const unsigned char* p = stage_ptr(nslot);
+      if (t + 1 < nst) read_b(p, t + 1);
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb) {
+        acc[mb] = mfma32(bf, af[mb], acc[mb]);
+        if (t + 1 < nst) af[mb] = read_a(p, 0, mb);
+      }
+      if (t + 1 < nst) bf = unpack_exact<false>(word(0), exact_scale(sc[0]), kr);
+    }
+    slot = nslot;
+    slot2 = slot2 == kPxTailRing - 1 ? 0 : slot2 + 1;
+  };
+  const std::integral_constant<int, 8> full;
+  const std::integral_constant<int, 4> half;
+  const std::integral_constant<int, 0> all;
+  auto no_hook = [] {};
+
+  __builtin_amdgcn_s_waitcnt(px_vm_wait(n));
+  px_barrier();  // the scales and stage 0 landed (stage 1 may still be loading)
+  if (work) {
+    read_b(stage_ptr(0), 0);
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) af[mb] = read_a(stage_ptr(0), 0, mb);
+    bf = unpack_exact<false>(word(0), exact_scale(sc[0]), kr);
+  }
+  for (int t = 0; t + 2 < nst; ++t)
+    stage(t, full, std::integral_constant<int, n>{}, [&](int sl) { px_issue_t<MBT>(a, lc, smem, t + 2, sl); }, no_hook);
+  // the last two stages refill nothing; the first of them brings the row
+  // indices (gate_up: the next item's rows, for its load sources; down: this
+  // item's output rows), the last takes the queue's next index
+  stage(nst - 2, full, std::integral_constant<int, 1>{}, [&](int) {
+    px_issue_table(a, smem, MODE == kModeGateUp && has_next ? nx.seg0 : it.seg0);
+  }, no_hook);
+  const bool fetch = fetch_q != nullptr && wave == 0;  // wavefront-uniform
+  int fv = 0;
+  auto take = [&](int) {
+    if (fetch && lane == 0) fv = __hip_atomic_fetch_add(fetch_q, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
+  auto put = [&] {
+    if (fetch && lane == 0) *reinterpret_cast<int*>(smem + kPxQSlot) = fv;
+  };
+  if (nkt & 1)
+    stage(nst - 1, half, all, take, put);
+  else
+    stage(nst - 1, full, all, take, put);
+  const int n_next = has_next ? px_issue_first<MODE, TILED>(a, nx, smem) : 0;
+  if (work) px_store<MODE, MB>(a, smem, it, wg, mo, acc);
+  return n_next;
+}
+
+template <int MODE, bool TILED>
 __device__ __forceinline__ int px_dispatch(const PrefillArgs& a, unsigned char* smem, const PxItem& it,
-                                           const PxItem& nx, bool has_next, int p0, int n_inflight,
-                                           int* fetch_q) {
-  if (it.nb > 1) return px_run_w<MODE>(a, smem, it, nx, has_next, p0, n_inflight, fetch_q);
+                                           const PxItem& nx, bool has_next, int n_inflight, int* fetch_q) {
+  if constexpr (TILED)
+    if (it.nb > 1) return px_run_w<MODE, TILED>(a, smem, it, nx, has_next, n_inflight, fetch_q);
+  // gate_up's half n-tile: eight wavefronts on four wavefronts' columns
+  const bool half = MODE == kModeGateUp && a.I - 128 * it.nt == 64;
+  if (px_is_tail<TILED>(a, it)) {
+    if constexpr (!TILED)
+      if (it.mb == 1) return px_run_t<MODE, TILED, 1>(a, smem, it, nx, has_next, fetch_q);
+    if constexpr (MODE == kModeGateUp)
+      if (half) return px_run_t<MODE, TILED, 1, 2>(a, smem, it, nx, has_next, fetch_q);
+    return px_run_t<MODE, TILED, 2>(a, smem, it, nx, has_next, fetch_q);
+  }
   if constexpr (MODE == kModeGateUp) {
-    if (a.I - 128 * it.nt == 64 && it.mb >= 2) {
-      // half n-tile: eight wavefronts on four wavefronts' columns
-      if (it.mb == 8) return px_run<MODE, 4, true>(a, smem, it, nx, has_next, p0, n_inflight, fetch_q);
-      if (it.mb == 4) return px_run<MODE, 2, true>(a, smem, it, nx, has_next, p0, n_inflight, fetch_q);
-      return px_run<MODE, 1, true>(a, smem, it, nx, has_next, p0, n_inflight, fetch_q);
+    if (half && it.mb >= 2) {
+      if (it.mb == 8) return px_run<MODE, TILED, 4, true>(a, smem, it, nx, has_next, n_inflight, fetch_q);
+      if (it.mb == 4) return px_run<MODE, TILED, 2, true>(a, smem, it, nx, has_next, n_inflight, fetch_q);
+      return px_run<MODE, TILED, 1, true>(a, smem, it, nx, has_next, n_inflight, fetch_q);
     }
   }
-  if (it.mb == 8) return px_run<MODE, 8>(a, smem, it, nx, has_next, p0, n_inflight, fetch_q);
-  if (it.mb == 4) return px_run<MODE, 4>(a, smem, it, nx, has_next, p0, n_inflight, fetch_q);
-  if (it.mb == 2) return px_run<MODE, 2>(a, smem, it, nx, has_next, p0, n_inflight, fetch_q);
-  return px_run<MODE, 1>(a, smem, it, nx, has_next, p0, n_inflight, fetch_q);
+  if (it.mb == 8) return px_run<MODE, TILED, 8>(a, smem, it, nx, has_next, n_inflight, fetch_q);
+  if (it.mb == 4) return px_run<MODE, TILED, 4>(a, smem, it, nx, has_next, n_inflight, fetch_q);
+  if (it.mb == 2) return px_run<MODE, TILED, 2>(a, smem, it, nx, has_next, n_inflight, fetch_q);
+  return px_run<MODE, TILED, 1>(a, smem, it, nx, has_next, n_inflight, fetch_q);
 }
 
 // Persistent grid, one workgroup per CU.  down: local item i of XCD x is
@@ -732,12 +993,14 @@ __device__ __forceinline__ int px_dispatch(const PrefillArgs& a, unsigned char* 
 // loaded during the current one).  queues[8] counts the workgroups that
 // have left; the expert sort zeroes the counters and the last workgroup to
 // leave resets them.  Without queues the deal is fixed: items b + r P.
-template <int MODE>
+template <int MODE, bool TILED>
 __global__ __launch_bounds__(kPxThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void k_prefill_x(PrefillArgs a) {
   extern __shared__ __align__(16) unsigned char smem[];
   const int ntiles = ld_uniform(a.counters, 1);
-  const int tiny0 = ld_uniform(a.counters, 2), tiny1 = ld_uniform(a.counters, 3);  // the smallest tails
+  // the tails that run as wide items (tiled weights)
+  const int tiny0 = TILED ? ld_uniform(a.counters, 2) : 0;
+  const int tiny1 = TILED ? ld_uniform(a.counters, 3) : 0;
   constexpr bool kChip = MODE == kModeGateUp;  // one queue for the chip
   const int x0 = kChip ? 0 : (int)(blockIdx.x & 7);
   const int xs = kChip ? 1 : 8;
@@ -764,7 +1027,6 @@ void k_prefill_x(PrefillArgs a) {
     leave();
     return;
   }
-  const int nkt = a.K / kPxKT;
   PxItem cur = px_item_info(a, x0, xs, t0, t1, n_wide, item);
   if (MODE == kModeGateUp) {
     // the first item's gathered rows into the table (nothing else in flight)
@@ -775,20 +1037,18 @@ void k_prefill_x(PrefillArgs a) {
     __builtin_amdgcn_s_waitcnt(px_vm_wait(0));
     px_barrier();
   }
-  int n_inflight = px_issue_first<MODE>(a, cur, smem, 0);
-  int p0 = 0;
+  int n_inflight = px_issue_first<MODE, TILED>(a, cur, smem);
   int nitem = item + P;
   for (;;) {
     const bool has_next = nitem < it_end;
     const PxItem nxt = has_next ? px_item_info(a, x0, xs, t0, t1, n_wide, nitem) : cur;
     // with a next item, take the index of the one after it during this item
-    n_inflight = px_dispatch<MODE>(a, smem, cur, nxt, has_next, p0, n_inflight, has_next ? queue : nullptr);
+    n_inflight = px_dispatch<MODE, TILED>(a, smem, cur, nxt, has_next, n_inflight, has_next ? queue : nullptr);
     if (!has_next) break;
     item = nitem;
     nitem = queue != nullptr ? 2 * P + __builtin_amdgcn_readfirstlane(*reinterpret_cast<volatile int*>(smem + kPxQSlot))
                              : item + P;
     cur = nxt;
-    p0 = (p0 + nkt) % kPxStages;
   }
   // the loads issued past the last stage land before the workgroup leaves
   __builtin_amdgcn_s_waitcnt(px_vm_wait(0));
@@ -874,17 +1134,33 @@ bool prefill_x_supported(int64_t H, int64_t I, int64_t G) {
 
 hipError_t launch_prefill_x(int mode, PrefillArgs a, int max_mtiles, hipStream_t s) {
   if (max_mtiles <= 0) return hipSuccess;
+  // tail items where the ring leaves room for the item's scales (gate_up's
+  // second block in the LDS that only down's epilogue uses if it fits there,
+  // else behind the first) and K has three stages of 128; else px_run's
+  // stages bring their own scales
+  const int sb = (((mode == kModeGateUp ? 128 : kPxBN) * a.ng * 2 + 16) + 1023) / 1024 * 1024;
+  for (int mbt = 1; mbt <= kPxTailMaxBlocks; ++mbt) {
+    const int s0 = kPxTailRing * px_tail_stage(mbt);
+    const bool apart = mode != kModeGateUp || sb <= kPxQSlot - kPxEpiOff;
+    a.tail_s1[mbt - 1] = mode != kModeGateUp ? 0 : apart ? kPxEpiOff : s0 + sb;
+    if (s0 + (apart ? 1 : 2) * sb > kPxTable || a.K <= 4 * kPxKT) a.tail_s1[mbt - 1] = -1;
+  }
   const size_t lds = prefill_x_lds_bytes();
+  auto launch = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3(prefill_grid_size(reinterpret_cast<const void*>(kern), kPxThreads, lds,
+                                                    max_mtiles * a.n_nt)),
+                       dim3(kPxThreads), lds, s, a);
+  };
   if (mode == kModeGateUp) {
-    auto kern = k_prefill_x<kModeGateUp>;
-    hipLaunchKernelGGL(kern, dim3(prefill_grid_size(reinterpret_cast<const void*>(kern), kPxThreads, lds,
-                                                    max_mtiles * a.n_nt)),
-                       dim3(kPxThreads), lds, s, a);
+    if (a.wt != nullptr)
+      launch(k_prefill_x<kModeGateUp, true>);
+    else
+      launch(k_prefill_x<kModeGateUp, false>);
   } else {
-    auto kern = k_prefill_x<kModeDown>;
-    hipLaunchKernelGGL(kern, dim3(prefill_grid_size(reinterpret_cast<const void*>(kern), kPxThreads, lds,
-                                                    max_mtiles * a.n_nt)),
-                       dim3(kPxThreads), lds, s, a);
+    if (a.wt != nullptr)
+      launch(k_prefill_x<kModeDown, true>);
+    else
+      launch(k_prefill_x<kModeDown, false>);
   }
   return hipGetLastError();
 }

@@ -98,6 +98,9 @@ struct PrefillArgs {
   // exact-form kernel, nullable: the weights' tiled copy (k_tile_prefill):
   // [E][n_nt][K/64][256 tile rows][32 B], each item's stage one 8 KiB block
   const int32_t* wt;
+  // exact-form kernel, set by the launcher: whether there are tail items of
+  // one and two m-blocks (-1: no), and where gate_up's up scales go in LDS
+  int tail_s1[2];
 };
 
 enum DecodeMode { kModeDense = 0, kModeGateUp = 1, kModeDown = 2 };
