@@ -80,11 +80,17 @@ struct AddNorm {
   uint16_t* y;
 };
 
-// Rows up to which the shared MLP's linears stream their weights
-// (k_linear_bf16, 64 rows per pass); above, the tiled GEMM.  FFN block (H =
-// 2816, Im = 2112) at 65 / 96 / 128 / 300 / 2048 rows: streamed 180 / 194 /
-// 244 / 331 / 1237 us, tiled 186 / 188 / 226 / 246 / 506 us.
-constexpr int64_t kLinearStreamMaxM = 80;
+// Whether a shared-MLP linear (M rows, N output columns, K deep) runs as the
+// tiled GEMM instead of streaming its weights once per 64 rows
+// (k_linear_bf16).  A launch of few tiles takes a tile's time, about 20 us at
+// K = 2816, whatever its size; the stream's time grows with the weights and
+// the 64-row passes.  The FFN block (H = 2816), streamed / tiled, in us: Im =
+// 1056 at 96 / 128 / 160 rows 170/182, 218/219, 228/223; Im = 1600 at 81 / 96
+// 178/179, 185/183; Im = 2112 at 65 / 81 / 300 / 2048 181/187, 187/186,
+// 331/246, 1237/506; Im = 4096 at 65 211/204.
+inline bool linear_tiled(int64_t M, int64_t N, int64_t K) {
+  return M > 64 && M * N * K > 420000000 && gemm_bf16_supported(K, N);
+}
 
 // The BF16 experts' routed rows up to which their weights stream once per
 // 16..64 rows of an expert (k_bf16_expert); above, the tiled GEMM (an
@@ -94,7 +100,7 @@ constexpr int64_t kLinearStreamMaxM = 80;
 constexpr int64_t kBf16StreamMaxRows = 192;
 
 inline hipError_t launch_linear_call(const LinearCall& l, hipStream_t s) {
-  if ((l.epi == kLinGateUp || l.epi == kLinPlain) && l.M > kLinearStreamMaxM && gemm_bf16_supported(l.K, l.N)) {
+  if ((l.epi == kLinGateUp || l.epi == kLinPlain) && linear_tiled(l.M, l.N, l.K)) {
     GemmBf16Args a{};
     a.act = l.x;
     a.W = l.W;

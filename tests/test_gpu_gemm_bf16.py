@@ -94,14 +94,14 @@ def test_bf16_experts_two_slots_and_invalid(dev, H, I):
     assert ((got - ref).abs() <= slack + 2.0 ** -8 * ref.abs()).all()
 
 
-# rows either side of the streaming kernel's range and of a tile, and (at Im = 2112: 17 column tiles) enough for
-# every tile height of the dense launch
-@pytest.mark.parametrize("M,Im", [(M, Im) for M in (80, 81, 96, 97, 161, 300) for Im in (192, 160)]
-                         + [(M, 2112) for M in (81, 480, 700, 1025, 1700, 2047)])
+# at H = 2816 the tiled GEMM takes more than 420e6 multiply-adds (M H Im): both sides of that, tiles' edges, half k
+# stages (Im % 64 == 32) and rows enough for every tile height of the dense launch
+@pytest.mark.parametrize("M,Im", [(65, 160), (81, 1056), (129, 1120), (193, 800), (257, 608), (300, 1056), (481, 2112),
+                                  (700, 2112), (1025, 2112), (1700, 2112), (2047, 2112)])
 def test_ffn_shared_mlp_rows(dev, M, Im):
     """The block with one expert whose weights are all zero (q = 0): its output is
     norm3(norm1(mlp) + 0), the shared MLP alone."""
-    H, I, E, G = 288, 192, 4, 32
+    H, I, E, G = 2816, 192, 4, 32
     g = torch.Generator(device=dev).manual_seed(31)
     lin = lambda o, i: (torch.randn(o, i, generator=g, device=dev) / math.sqrt(i)).to(torch.bfloat16)
     one = torch.ones(H, dtype=torch.bfloat16, device=dev)
