@@ -92,6 +92,14 @@ inline bool linear_tiled(int64_t M, int64_t N, int64_t K) {
   return M > 64 && M * N * K > 420000000 && gemm_bf16_supported(K, N);
 }
 
+// Whether Linear4Bit (M rows, N columns) runs as the tiled GEMM instead of
+// streaming its weights once per 16 rows (k_decode<dense>).  Few tiles take a
+// tile's time, which grows with K as the stream's does.  K = 2816, streamed /
+// tiled, in us: N = 2816 at 256 / 384 / 2048 rows 21/24, 30/24, 99/40 (G = 32;
+// 20/25, 27/26, 90/40 at G = 128); N = 1408 at 512 / 768 rows 21/24, 30/24;
+// K = 1056, N = 704 at 1024 / 1536 rows 16/16, 21/16.
+inline bool linear_w4_tiled(int64_t M, int64_t N) { return M > 64 && M * N > 900000; }
+
 // The BF16 experts' routed rows up to which their weights stream once per
 // 16..64 rows of an expert (k_bf16_expert); above, the tiled GEMM (an
 // expert's weights once per 128 rows).  Gemma shape at 128 / 256 / 512 / 8248
@@ -323,6 +331,8 @@ int w4a16_linear(const uint16_t* x, const int32_t* w_packed, const uint16_t* w_s
   (void)workspace_bytes;
   if (K > kMaxStreamK) return W4A16_ERR_SHAPE;
   hipStream_t s = static_cast<hipStream_t>(stream);
+  if (linear_w4_tiled(M, N) && linear_w4_supported(M, N, K, group_size))
+    return launch_status(launch_linear_w4(x, w_packed, w_scale, bias, y, M, N, K, group_size, s));
   DecodeArgs a{};
   a.act = x;
   a.wp = w_packed;
