@@ -163,7 +163,7 @@ __device__ __forceinline__ PxItem px_item_info(const PrefillArgs& a, int x0, int
   it.e = tile >> 16;
   it.seg0 = ld_uniform(a.offsets, it.e) + (tile & 0xFFFF) * kPxBM;
   it.nrows = min(kPxBM, ld_uniform(a.offsets, it.e + 1) - it.seg0);
-  it.mb = it.nrows > 128 ? 8 : it.nrows > 64 ? 4 : it.nrows > 32 ? 2 : 1;
+  it.mb = (it.nrows + 31) >> 5;  // 32-row blocks
   return it;
 }
 
@@ -965,15 +965,22 @@ __device__ __forceinline__ int px_dispatch(const PrefillArgs& a, unsigned char* 
   }
   if constexpr (MODE == kModeGateUp) {
     if (half && it.mb >= 2) {
-      if (it.mb == 8) return px_run<MODE, TILED, 4, true>(a, smem, it, nx, has_next, n_inflight, fetch_q);
-      if (it.mb == 4) return px_run<MODE, TILED, 2, true>(a, smem, it, nx, has_next, n_inflight, fetch_q);
+      if (it.mb >= 7) return px_run<MODE, TILED, 4, true>(a, smem, it, nx, has_next, n_inflight, fetch_q);
+      if (it.mb >= 5) return px_run<MODE, TILED, 3, true>(a, smem, it, nx, has_next, n_inflight, fetch_q);
+      if (it.mb >= 3) return px_run<MODE, TILED, 2, true>(a, smem, it, nx, has_next, n_inflight, fetch_q);
       return px_run<MODE, TILED, 1, true>(a, smem, it, nx, has_next, n_inflight, fetch_q);
     }
   }
-  if (it.mb == 8) return px_run<MODE, TILED, 8>(a, smem, it, nx, has_next, n_inflight, fetch_q);
-  if (it.mb == 4) return px_run<MODE, TILED, 4>(a, smem, it, nx, has_next, n_inflight, fetch_q);
-  if (it.mb == 2) return px_run<MODE, TILED, 2>(a, smem, it, nx, has_next, n_inflight, fetch_q);
-  return px_run<MODE, TILED, 1>(a, smem, it, nx, has_next, n_inflight, fetch_q);
+  switch (it.mb) {
+    case 8: return px_run<MODE, TILED, 8>(a, smem, it, nx, has_next, n_inflight, fetch_q);
+    case 7: return px_run<MODE, TILED, 7>(a, smem, it, nx, has_next, n_inflight, fetch_q);
+    case 6: return px_run<MODE, TILED, 6>(a, smem, it, nx, has_next, n_inflight, fetch_q);
+    case 5: return px_run<MODE, TILED, 5>(a, smem, it, nx, has_next, n_inflight, fetch_q);
+    case 4: return px_run<MODE, TILED, 4>(a, smem, it, nx, has_next, n_inflight, fetch_q);
+    case 3: return px_run<MODE, TILED, 3>(a, smem, it, nx, has_next, n_inflight, fetch_q);
+    case 2: return px_run<MODE, TILED, 2>(a, smem, it, nx, has_next, n_inflight, fetch_q);
+    default: return px_run<MODE, TILED, 1>(a, smem, it, nx, has_next, n_inflight, fetch_q);
+  }
 }
 
 // Persistent grid, one workgroup per CU.  down: local item i of XCD x is
