@@ -64,6 +64,7 @@ struct DecodeArgs {
   // slot arithmetic for it (workgroups per slot, its division magic, items
   // per workgroup)
   int u_guess, wps_guess, per_guess;
+  int resident;     // workgroups that run at once when the grid holds more (0: it does not)
   uint32_t slot_magic;
   // the gate_up launch's own plan (launch_decode's self_args / self_mode):
   // the top-k + sort's arguments (kSelfPlan: idx_out is the finished top-k
