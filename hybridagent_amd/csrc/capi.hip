@@ -107,6 +107,13 @@ inline bool linear_w4_tiled(int64_t M, int64_t N) { return M > 64 && M * N > 900
 // with Zipf-skewed routing 135 / 202 / 335 us against 142 / 158 / 231.
 constexpr int64_t kBf16StreamMaxRows = 192;
 
+// The FFN block's last launch (launch_ffn_post), run by the layer in place of
+// its combine where it has one (done: it was).
+struct FfnPost {
+  FfnPostCall call;
+  bool done;
+};
+
 inline hipError_t launch_linear_call(const LinearCall& l, hipStream_t s) {
   if ((l.epi == kLinGateUp || l.epi == kLinPlain) && linear_tiled(l.M, l.N, l.K)) {
     GemmBf16Args a{};
@@ -747,11 +754,20 @@ constexpr int64_t kFuseDownCombineRows = 32;
 int down_and_combine(const int32_t* dn_packed, const uint16_t* dn_scale, const int64_t* topk_idx,
                      const float* topk_w, uint16_t* out, int64_t M, int64_t top_k, int64_t E,
                      int64_t H, int64_t I, int64_t group_size, void* workspace,
-                     size_t workspace_bytes, void* stream, const Tiles& t, const AddNorm* an = nullptr) {
+                     size_t workspace_bytes, void* stream, const Tiles& t, const AddNorm* an = nullptr,
+                     FfnPost* post = nullptr) {
   if (use_prefill(M, H, I) || M * top_k > kFuseDownCombineRows || !down_combine_supported(M, top_k, I)) {
     int st = down_impl(dn_packed, dn_scale, t, M, top_k, E, H, I, group_size, workspace, workspace_bytes,
                        stream);
     if (st != W4A16_OK) return st;
+    if (post != nullptr && ffn_post_combines(top_k)) {
+      MoeLayout L{};
+      st = moe_check(M, top_k, E, H, I, group_size, workspace, workspace_bytes, &L);
+      if (st != W4A16_OK) return st;
+      post->done = true;
+      return launch_status(launch_ffn_post(post->call, L.dn, topk_idx, topk_w, (int)top_k, (int)E, M, (int)H,
+                                           static_cast<hipStream_t>(stream)));
+    }
     if (an != nullptr && top_k <= 8) {
       MoeLayout L{};
       st = moe_check(M, top_k, E, H, I, group_size, workspace, workspace_bytes, &L);
@@ -903,7 +919,7 @@ static int layer_forward_impl(const uint16_t* router_in, const uint16_t* router_
                               uint16_t* out, int64_t* topk_idx, float* topk_w, int64_t M, int64_t top_k,
                               int64_t E, int64_t H, int64_t I, int64_t group_size, void* workspace,
                               size_t workspace_bytes, void* stream, const SharedMlp* mlp = nullptr,
-                              const AddNorm* an = nullptr);
+                              const AddNorm* an = nullptr, FfnPost* post = nullptr);
 
 static int ffn_block_impl(const uint16_t* residual, const uint16_t* attn_out,
                           const uint16_t* post_attn_ln_w, const uint16_t* pre_ff_ln_w,
@@ -949,12 +965,12 @@ static int ffn_block_impl(const uint16_t* residual, const uint16_t* attn_out,
                                  (int)H},
                       LinearCall{kLinPlain, L.inter, mlp_down_w, nullptr, nullptr, nullptr, L.h_mlp, M, (int)H,
                                  (int)Im}};
+  FfnPost post{FfnPostCall{L.h_mlp, L.res, post_ff_ln1_w, post_ff_ln2_w, post_ff_ln_w, layer_scalar, out, eps}, false};
   st = layer_forward_impl(L.res, router_scale, router_scalar_root, router_proj_w, router_per_expert_scale, eps,
                           L.h2_in, gu_packed, gu_scale, dn_packed, dn_scale, t, L.moe, L.idx, L.w, M, top_k, E, H,
-                          I, group_size, L.moe_ws, L.moe_bytes, stream, &mlp);
-  if (st != W4A16_OK) return st;
-  return launch_status(launch_ffn_post(L.h_mlp, L.moe, L.res, post_ff_ln1_w, post_ff_ln2_w, post_ff_ln_w,
-                                       layer_scalar, out, M, (int)H, eps, s));
+                          I, group_size, L.moe_ws, L.moe_bytes, stream, &mlp, nullptr, &post);
+  if (st != W4A16_OK || post.done) return st;
+  return launch_status(launch_ffn_post(post.call, L.moe, nullptr, nullptr, 0, 0, M, (int)H, s));
 }
 
 int moe_ffn_block_forward(const uint16_t* residual, const uint16_t* attn_out,
@@ -1167,7 +1183,8 @@ static int layer_forward_impl(const uint16_t* router_in, const uint16_t* router_
                               const int32_t* dn_packed, const uint16_t* dn_scale, const Tiles& t,
                               uint16_t* out, int64_t* topk_idx, float* topk_w, int64_t M, int64_t top_k,
                               int64_t E, int64_t H, int64_t I, int64_t group_size, void* workspace,
-                              size_t workspace_bytes, void* stream, const SharedMlp* mlp, const AddNorm* an) {
+                              size_t workspace_bytes, void* stream, const SharedMlp* mlp, const AddNorm* an,
+                              FfnPost* post) {
   if (M < 0 || M > (1 << 24) || top_k > E) return W4A16_ERR_SHAPE;
   if (M == 0) {
     MoeLayout dummy{};
@@ -1217,7 +1234,7 @@ static int layer_forward_impl(const uint16_t* router_in, const uint16_t* router_
                       &ta, kSelfRoute);
     if (st == W4A16_OK)
       st = down_and_combine(dn_packed, dn_scale, topk_idx, topk_w, out, M, top_k, E, H, I, group_size, workspace,
-                            moe_bytes, stream, t, an);
+                            moe_bytes, stream, t, an, post);
     return st;
   }
   if (M * top_k <= kTopkSortMaxEntries) {
@@ -1254,7 +1271,7 @@ static int layer_forward_impl(const uint16_t* router_in, const uint16_t* router_
                         &ta, kSelfPlan);
       if (st == W4A16_OK)
         return down_and_combine(dn_packed, dn_scale, topk_idx, topk_w, out, M, top_k, E, H, I, group_size,
-                                workspace, moe_bytes, stream, t, an);
+                                workspace, moe_bytes, stream, t, an, post);
     }
     st = moe_plan(hidden, topk_idx, M, top_k, E, H, I, group_size, workspace, moe_bytes, stream);
     if (st != W4A16_OK) return st;
@@ -1264,7 +1281,7 @@ static int layer_forward_impl(const uint16_t* router_in, const uint16_t* router_
                     moe_bytes, stream);
   if (st == W4A16_OK)
     st = down_and_combine(dn_packed, dn_scale, topk_idx, topk_w, out, M, top_k, E, H, I,
-                          group_size, workspace, moe_bytes, stream, t, an);
+                          group_size, workspace, moe_bytes, stream, t, an, post);
   return st;
 }
 

@@ -6,7 +6,10 @@
 //               res    = bf16(residual + h)                         (:103)
 //               h_ff   = rms_norm(res) * pre_ff_ln_w                (:105)
 //               h2_in  = rms_norm(res) * pre_ff_ln2_w               (:119)
-//   k_ffn_post  h_1    = rms_norm(h_mlp) * post_ff_ln1_w            (:109)
+//   k_ffn_post  moe_out = sum_j bf16(bf16(w[t, j]) dn[t k + j])     (:121-122,
+//               KMAX > 0: k_combine's arithmetic, without the row's round
+//               trip through memory and its launch)
+//               h_1    = rms_norm(h_mlp) * post_ff_ln1_w            (:109)
 //               h_2    = rms_norm(moe_out) * post_ff_ln2_w          (:123)
 //               h_comb = rms_norm(bf16(h_1 + h_2)) * post_ff_ln_w   (:125)
 //               out    = bf16(bf16(res + h_comb) * layer_scalar)    (:126)
@@ -24,7 +27,13 @@ namespace w4a16 {
 namespace {
 
 constexpr int kFfnThreads = 256;
-constexpr int kFfnChunks = 4;  // 16-byte chunks per thread: H <= 256 * 4 * 8
+// 16-byte chunks per thread, at most: H <= 256 * 4 * 8.  The kernels are built
+// for NQ = 1 .. 4 of them: with the registers of four a row of 2816 (NQ = 2)
+// kept half the rows in flight (2048 rows: pre 17.8 -> 14.5 us, combine and
+// post 18.3 + 17.7 -> 32.5 us in one launch).
+constexpr int kFfnChunks = 4;
+// most slots the combine inside k_ffn_post takes
+constexpr int kFfnTopK = 8;
 
 // sums of two values over the workgroup in a fixed order
 __device__ __forceinline__ float2 block_sum2(float a, float b, float2* part) {
@@ -97,6 +106,7 @@ __device__ __forceinline__ void norm8(const Row8& x, float rstd, const Row8& w, 
 
 }  // namespace
 
+template <int NQ>
 __global__ __launch_bounds__(kFfnThreads) void k_ffn_pre(
     const uint16_t* __restrict__ attn, const uint16_t* __restrict__ res, const uint16_t* __restrict__ w_pa,
     const uint16_t* __restrict__ w_pf, const uint16_t* __restrict__ w_pf2, uint16_t* __restrict__ res_out,
@@ -104,18 +114,18 @@ __global__ __launch_bounds__(kFfnThreads) void k_ffn_pre(
   __shared__ float2 part[kFfnThreads / 64];
   const int64_t off = (int64_t)blockIdx.x * H;
   const int n8 = H >> 3;
-  Row8 a[kFfnChunks], r[kFfnChunks];
+  Row8 a[NQ], r[NQ];
   // every load issued before the first reduction: the rows, then the three
   // norms' weights (one memory round trip instead of three)
-  u32x4_t wa[kFfnChunks], wf[kFfnChunks], wf2[kFfnChunks];
+  u32x4_t wa[NQ], wf[NQ], wf2[NQ];
 #pragma unroll
-  for (int q = 0; q < kFfnChunks; ++q) {
+  for (int q = 0; q < NQ; ++q) {
     const int c8 = threadIdx.x + kFfnThreads * q;
     a[q] = load8(attn + off, c8, c8 < n8);
     r[q] = load8(res + off, c8, c8 < n8);
   }
 #pragma unroll
-  for (int q = 0; q < kFfnChunks; ++q) {
+  for (int q = 0; q < NQ; ++q) {
     const int c8 = threadIdx.x + kFfnThreads * q;
     wa[q] = raw8(w_pa, c8, c8 < n8);
     wf[q] = raw8(w_pf, c8, c8 < n8);
@@ -123,11 +133,11 @@ __global__ __launch_bounds__(kFfnThreads) void k_ffn_pre(
   }
   float ssa = 0.f;
 #pragma unroll
-  for (int q = 0; q < kFfnChunks; ++q) ssa += sumsq8(a[q]);
+  for (int q = 0; q < NQ; ++q) ssa += sumsq8(a[q]);
   const float rsa = 1.0f / sqrtf(block_sum2(ssa, 0.f, part).x / (float)H + eps);
   float ssr = 0.f;
 #pragma unroll
-  for (int q = 0; q < kFfnChunks; ++q) {
+  for (int q = 0; q < NQ; ++q) {
     const int c8 = threadIdx.x + kFfnThreads * q;
     const bool ok = c8 < n8;
     const Row8 w = conv8(wa[q]);
@@ -140,7 +150,7 @@ __global__ __launch_bounds__(kFfnThreads) void k_ffn_pre(
   }
   const float rsr = 1.0f / sqrtf(block_sum2(ssr, 0.f, part).x / (float)H + eps);
 #pragma unroll
-  for (int q = 0; q < kFfnChunks; ++q) {
+  for (int q = 0; q < NQ; ++q) {
     const int c8 = threadIdx.x + kFfnThreads * q;
     if (c8 >= n8) continue;
     float o[8];
@@ -151,25 +161,48 @@ __global__ __launch_bounds__(kFfnThreads) void k_ffn_pre(
   }
 }
 
+template <int NQ, int KMAX>
 __global__ __launch_bounds__(kFfnThreads) void k_ffn_post(
     const uint16_t* __restrict__ mlp, const uint16_t* __restrict__ moe, const uint16_t* __restrict__ res,
     const uint16_t* __restrict__ w1, const uint16_t* __restrict__ w2, const uint16_t* __restrict__ w3,
-    const uint16_t* __restrict__ layer_scalar, uint16_t* __restrict__ out, int H, float eps) {
+    const uint16_t* __restrict__ layer_scalar, uint16_t* __restrict__ out, int H, float eps,
+    const int64_t* __restrict__ idx, const float* __restrict__ tw, int topk, int E) {
   __shared__ float2 part[kFfnThreads / 64];
   const int64_t off = (int64_t)blockIdx.x * H;
   const int n8 = H >> 3;
-  Row8 m[kFfnChunks], e2[kFfnChunks];
+  Row8 m[NQ], e2[NQ];
+  // KMAX > 0: moe holds the expert rows t * topk + j; every slot's index,
+  // weight and chunks are requested before the first is used
+  constexpr int KM = KMAX > 0 ? KMAX : 1;
+  const int64_t r0 = (int64_t)blockIdx.x * topk;
+  int64_t ex[KM];
+  float wv[KM];
+  u32x4_t d[NQ][KM];
+  if (KMAX > 0) {
+#pragma unroll
+    for (int j = 0; j < KM; ++j) {
+      const int64_t r = r0 + (j < topk ? j : 0);
+      ex[j] = idx[r];
+      wv[j] = tw[r];
+    }
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+      const int c8 = threadIdx.x + kFfnThreads * q;
+#pragma unroll
+      for (int j = 0; j < KM; ++j) d[q][j] = raw8(moe + (r0 + j) * H, c8, c8 < n8 && j < topk);
+    }
+  }
   // every load issued before the first reduction: the two rows, then the
   // three norms' weights and the residual row (one memory round trip)
-  u32x4_t w1r[kFfnChunks], w2r[kFfnChunks], w3r[kFfnChunks], rr[kFfnChunks];
+  u32x4_t w1r[NQ], w2r[NQ], w3r[NQ], rr[NQ];
 #pragma unroll
-  for (int q = 0; q < kFfnChunks; ++q) {
+  for (int q = 0; q < NQ; ++q) {
     const int c8 = threadIdx.x + kFfnThreads * q;
     m[q] = load8(mlp + off, c8, c8 < n8);
-    e2[q] = load8(moe + off, c8, c8 < n8);
+    if (KMAX == 0) e2[q] = load8(moe + off, c8, c8 < n8);
   }
 #pragma unroll
-  for (int q = 0; q < kFfnChunks; ++q) {
+  for (int q = 0; q < NQ; ++q) {
     const int c8 = threadIdx.x + kFfnThreads * q;
     w1r[q] = raw8(w1, c8, c8 < n8);
     w2r[q] = raw8(w2, c8, c8 < n8);
@@ -177,9 +210,27 @@ __global__ __launch_bounds__(kFfnThreads) void k_ffn_post(
     rr[q] = raw8(res + off, c8, c8 < n8);
   }
   const float ls = bf16_bits_to_f32(layer_scalar[0]);
+  if (KMAX > 0) {
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+      float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < KM; ++j) {
+        if (j < topk && ex[j] >= 0 && ex[j] < E) {
+          const float wb = round_bf16(wv[j]);
+          const Row8 r = conv8(d[q][j]);
+#pragma unroll
+          for (int t = 0; t < 8; ++t) acc[t] += round_bf16(r.v[t] * wb);
+        }
+      }
+      const bool ok = threadIdx.x + kFfnThreads * q < n8;
+#pragma unroll
+      for (int t = 0; t < 8; ++t) e2[q].v[t] = ok ? round_bf16(acc[t]) : 0.f;
+    }
+  }
   float ssm = 0.f, sse = 0.f;
 #pragma unroll
-  for (int q = 0; q < kFfnChunks; ++q) {
+  for (int q = 0; q < NQ; ++q) {
     ssm += sumsq8(m[q]);
     sse += sumsq8(e2[q]);
   }
@@ -189,7 +240,7 @@ __global__ __launch_bounds__(kFfnThreads) void k_ffn_post(
   // c = bf16(h_1 + h_2), kept in m[]
   float ssc = 0.f;
 #pragma unroll
-  for (int q = 0; q < kFfnChunks; ++q) {
+  for (int q = 0; q < NQ; ++q) {
     const int c8 = threadIdx.x + kFfnThreads * q;
     const bool ok = c8 < n8;
     float h1[8], h2[8];
@@ -201,7 +252,7 @@ __global__ __launch_bounds__(kFfnThreads) void k_ffn_post(
   }
   const float rc = 1.0f / sqrtf(block_sum2(ssc, 0.f, part).x / (float)H + eps);
 #pragma unroll
-  for (int q = 0; q < kFfnChunks; ++q) {
+  for (int q = 0; q < NQ; ++q) {
     const int c8 = threadIdx.x + kFfnThreads * q;
     if (c8 >= n8) continue;
     float hc[8];
@@ -219,19 +270,43 @@ hipError_t launch_ffn_pre(const uint16_t* attn, const uint16_t* res, const uint1
                           uint16_t* h2_in, int64_t M, int H, float eps, hipStream_t s) {
   if (M == 0) return hipSuccess;
   if (H % 8 != 0 || H > kFfnThreads * kFfnChunks * 8) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_ffn_pre, dim3((unsigned)M), dim3(kFfnThreads), 0, s, attn, res, w_pa, w_pf, w_pf2,
-                     res_out, h_ff, h2_in, H, eps);
+  const dim3 grid((unsigned)M), block(kFfnThreads);
+#define W4A16_PRE(NQ_) \
+  hipLaunchKernelGGL(k_ffn_pre<NQ_>, grid, block, 0, s, attn, res, w_pa, w_pf, w_pf2, res_out, h_ff, h2_in, H, eps)
+  switch ((H / 8 + kFfnThreads - 1) / kFfnThreads) {
+    case 1: W4A16_PRE(1); break;
+    case 2: W4A16_PRE(2); break;
+    case 3: W4A16_PRE(3); break;
+    default: W4A16_PRE(4); break;
+  }
+#undef W4A16_PRE
   return hipGetLastError();
 }
 
-hipError_t launch_ffn_post(const uint16_t* mlp, const uint16_t* moe, const uint16_t* res,
-                           const uint16_t* w1, const uint16_t* w2, const uint16_t* w3,
-                           const uint16_t* layer_scalar, uint16_t* out, int64_t M, int H, float eps,
-                           hipStream_t s) {
+bool ffn_post_combines(int64_t topk) { return topk <= kFfnTopK; }
+
+hipError_t launch_ffn_post(const FfnPostCall& c, const uint16_t* moe, const int64_t* idx, const float* tw, int topk,
+                           int E, int64_t M, int H, hipStream_t s) {
   if (M == 0) return hipSuccess;
-  if (H % 8 != 0 || H > kFfnThreads * kFfnChunks * 8) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_ffn_post, dim3((unsigned)M), dim3(kFfnThreads), 0, s, mlp, moe, res, w1, w2, w3,
-                     layer_scalar, out, H, eps);
+  if (H % 8 != 0 || H > kFfnThreads * kFfnChunks * 8 || (idx != nullptr && !ffn_post_combines(topk)))
+    return hipErrorInvalidValue;
+  const dim3 grid((unsigned)M), block(kFfnThreads);
+#define W4A16_POST(NQ_, K_)                                                                                       \
+  hipLaunchKernelGGL((k_ffn_post<NQ_, K_>), grid, block, 0, s, c.mlp, moe, c.res, c.w1, c.w2, c.w3,               \
+                     c.layer_scalar, c.out, H, c.eps, idx, tw, topk, E)
+#define W4A16_POST2(NQ_)                          \
+  do {                                            \
+    if (idx != nullptr) W4A16_POST(NQ_, kFfnTopK); \
+    else W4A16_POST(NQ_, 0);                      \
+  } while (0)
+  switch ((H / 8 + kFfnThreads - 1) / kFfnThreads) {
+    case 1: W4A16_POST2(1); break;
+    case 2: W4A16_POST2(2); break;
+    case 3: W4A16_POST2(3); break;
+    default: W4A16_POST2(4); break;
+  }
+#undef W4A16_POST2
+#undef W4A16_POST
   return hipGetLastError();
 }
 

@@ -19,7 +19,9 @@ namespace w4a16 {
 namespace {
 
 constexpr int kLnThreads = 256;
-constexpr int kLnChunks = 4;  // H <= 256 * 8 * 4 = 8192 held in registers
+// 16-byte chunks per thread, at most: H <= 256 * 8 * 4 = 8192 held in registers
+// (the kernel is built for NQ = 1 .. 4: a row of 2816 takes two)
+constexpr int kLnChunks = 4;
 
 // sum over the workgroup in a fixed order (wave sums, then waves in order)
 __device__ __forceinline__ float block_sum(float v, float* part) {
@@ -39,7 +41,7 @@ __device__ __forceinline__ float block_sum(float v, float* part) {
 // nn.LayerNorm over rows of H (fp32 statistics, two passes: mean, then the
 // mean of squared deviations), affine with bf16 weight / bias, bf16 out
 // (FRAG: in the bf16 linears' fragment order, rows padded to 16).
-template <bool FRAG>
+template <bool FRAG, int NQ>
 __global__ __launch_bounds__(kLnThreads) void k_layer_norm(const uint16_t* __restrict__ x,
                                                           const uint16_t* __restrict__ w,
                                                           const uint16_t* __restrict__ b,
@@ -49,25 +51,25 @@ __global__ __launch_bounds__(kLnThreads) void k_layer_norm(const uint16_t* __res
   const int64_t row = blockIdx.x;
   const uint16_t* xr = x + row * H;
   const int n8 = H >> 3;
-  float v[kLnChunks][8];
+  float v[NQ][8];
   float s = 0.f;
   // the row, then the affine parameters, all loads issued before the first
   // is used: one memory round trip, and the statistics wait only for the
   // row (loads complete in order)
-  u32x4_t xv[kLnChunks], wv[kLnChunks], bv[kLnChunks];
+  u32x4_t xv[NQ], wv[NQ], bv[NQ];
 #pragma unroll
-  for (int q = 0; q < kLnChunks; ++q) {
+  for (int q = 0; q < NQ; ++q) {
     const int c8 = threadIdx.x + kLnThreads * q;
     xv[q] = c8 < n8 ? ld16(xr + 8 * c8) : u32x4_t{0u, 0u, 0u, 0u};
   }
 #pragma unroll
-  for (int q = 0; q < kLnChunks; ++q) {
+  for (int q = 0; q < NQ; ++q) {
     const int c8 = min(threadIdx.x + kLnThreads * q, n8 - 1);
     wv[q] = ld16(w + 8 * c8);
     bv[q] = ld16(b + 8 * c8);
   }
 #pragma unroll
-  for (int q = 0; q < kLnChunks; ++q) {
+  for (int q = 0; q < NQ; ++q) {
     const u32x4_t u = xv[q];
     const uint32_t w4[4] = {u.x, u.y, u.z, u.w};
 #pragma unroll
@@ -81,7 +83,7 @@ __global__ __launch_bounds__(kLnThreads) void k_layer_norm(const uint16_t* __res
   const float mean = block_sum(s, part) / (float)H;
   float d2 = 0.f;
 #pragma unroll
-  for (int q = 0; q < kLnChunks; ++q) {
+  for (int q = 0; q < NQ; ++q) {
     const int c8 = threadIdx.x + kLnThreads * q;
     if (c8 < n8) {
 #pragma unroll
@@ -93,7 +95,7 @@ __global__ __launch_bounds__(kLnThreads) void k_layer_norm(const uint16_t* __res
   }
   const float rstd = 1.0f / sqrtf(block_sum(d2, part) / (float)H + eps);
 #pragma unroll
-  for (int q = 0; q < kLnChunks; ++q) {
+  for (int q = 0; q < NQ; ++q) {
     const int c8 = threadIdx.x + kLnThreads * q;
     if (c8 < n8) {
       const uint32_t ww[4] = {wv[q].x, wv[q].y, wv[q].z, wv[q].w};
@@ -116,10 +118,21 @@ hipError_t launch_layer_norm(const uint16_t* x, const uint16_t* w, const uint16_
                              int64_t M, int H, float eps, bool frag, hipStream_t s) {
   if (M == 0) return hipSuccess;
   if (H % 8 != 0 || H > kLnThreads * 8 * kLnChunks || (frag && H % 32 != 0)) return hipErrorInvalidValue;
-  if (frag)
-    hipLaunchKernelGGL(k_layer_norm<true>, dim3((unsigned)M), dim3(kLnThreads), 0, s, x, w, b, y, H, eps);
-  else
-    hipLaunchKernelGGL(k_layer_norm<false>, dim3((unsigned)M), dim3(kLnThreads), 0, s, x, w, b, y, H, eps);
+  const dim3 grid((unsigned)M), block(kLnThreads);
+#define W4A16_LN(NQ_)                                                                              \
+  do {                                                                                             \
+    if (frag)                                                                                      \
+      hipLaunchKernelGGL((k_layer_norm<true, NQ_>), grid, block, 0, s, x, w, b, y, H, eps);        \
+    else                                                                                           \
+      hipLaunchKernelGGL((k_layer_norm<false, NQ_>), grid, block, 0, s, x, w, b, y, H, eps);       \
+  } while (0)
+  switch ((H / 8 + kLnThreads - 1) / kLnThreads) {
+    case 1: W4A16_LN(1); break;
+    case 2: W4A16_LN(2); break;
+    case 3: W4A16_LN(3); break;
+    default: W4A16_LN(4); break;
+  }
+#undef W4A16_LN
   return hipGetLastError();
 }
 

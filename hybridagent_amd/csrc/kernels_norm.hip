@@ -12,8 +12,11 @@
 namespace w4a16 {
 
 constexpr int kNormThreads = 256;
-constexpr int kNormChunks = 4;  // 16-byte chunks per thread: H <= 256 * 4 * 8
+// 16-byte chunks per thread, at most: H <= 256 * 4 * 8 (the kernels are built
+// for NQ = 1 .. 4: a row of 2816 takes two)
+constexpr int kNormChunks = 4;
 
+template <int NQ>
 __global__ __launch_bounds__(kNormThreads) void k_add_rms_norm(
     const uint16_t* __restrict__ h, const uint16_t* __restrict__ delta,
     const uint16_t* __restrict__ w, uint16_t* __restrict__ h_out, uint16_t* __restrict__ y,
@@ -24,9 +27,9 @@ __global__ __launch_bounds__(kNormThreads) void k_add_rms_norm(
   const int n8 = H >> 3;
   const uint16_t* hr = h + row * H;
   const uint16_t* dr = delta != nullptr ? delta + row * H : nullptr;
-  u32x4_t xv[kNormChunks], dv[kNormChunks];
+  u32x4_t xv[NQ], dv[NQ];
 #pragma unroll
-  for (int q = 0; q < kNormChunks; ++q) {
+  for (int q = 0; q < NQ; ++q) {
     const int c8 = tid + kNormThreads * q;
     xv[q] = u32x4_t{0u, 0u, 0u, 0u};
     dv[q] = u32x4_t{0u, 0u, 0u, 0u};
@@ -37,7 +40,7 @@ __global__ __launch_bounds__(kNormThreads) void k_add_rms_norm(
   }
   float ss = 0.f;
 #pragma unroll
-  for (int q = 0; q < kNormChunks; ++q) {
+  for (int q = 0; q < NQ; ++q) {
     const int c8 = tid + kNormThreads * q;
     if (c8 >= n8) continue;
     const uint32_t x4[4] = {xv[q].x, xv[q].y, xv[q].z, xv[q].w};
@@ -66,7 +69,7 @@ __global__ __launch_bounds__(kNormThreads) void k_add_rms_norm(
   for (int i = 0; i < kNormThreads / 64; ++i) tot += s_part[i];
   const float r = 1.0f / sqrtf(tot / (float)H + eps);
 #pragma unroll
-  for (int q = 0; q < kNormChunks; ++q) {
+  for (int q = 0; q < NQ; ++q) {
     const int c8 = tid + kNormThreads * q;
     if (c8 >= n8) continue;
     const u32x4_t wv = ld16(w + 8 * c8);
@@ -96,6 +99,7 @@ __global__ __launch_bounds__(kNormThreads) void k_add_rms_norm(
 //   out = combine(...)[t], h_out = bf16(h + out), y = bf16((h_out * r) * w)
 // topk <= 8; every load of the row (its k down-projection pieces, h and
 // the norm weight) is issued before the first is used.
+template <int NQ>
 __global__ __launch_bounds__(kNormThreads) void k_combine_add_rms_norm(
     const uint16_t* __restrict__ dn, const int64_t* __restrict__ idx, const float* __restrict__ tw,
     const uint16_t* __restrict__ h, const uint16_t* __restrict__ w, uint16_t* __restrict__ out,
@@ -114,9 +118,9 @@ __global__ __launch_bounds__(kNormThreads) void k_combine_add_rms_norm(
     ex[j] = idx[r];
     wv[j] = tw[r];
   }
-  u32x4_t d[kNormChunks][KMAX], hv[kNormChunks], gv[kNormChunks];
+  u32x4_t d[NQ][KMAX], hv[NQ], gv[NQ];
 #pragma unroll
-  for (int q = 0; q < kNormChunks; ++q) {
+  for (int q = 0; q < NQ; ++q) {
     const int c8 = min(tid + kNormThreads * q, n8 - 1);
 #pragma unroll
     for (int j = 0; j < KMAX; ++j) d[q][j] = ld16(dn + (r0 + (j < topk ? j : 0)) * H + 8 * c8);
@@ -124,9 +128,9 @@ __global__ __launch_bounds__(kNormThreads) void k_combine_add_rms_norm(
     gv[q] = ld16(w + 8 * c8);
   }
   float ss = 0.f;
-  u32x4_t xv[kNormChunks];
+  u32x4_t xv[NQ];
 #pragma unroll
-  for (int q = 0; q < kNormChunks; ++q) {
+  for (int q = 0; q < NQ; ++q) {
     const int c8 = tid + kNormThreads * q;
     xv[q] = u32x4_t{0u, 0u, 0u, 0u};
     if (c8 >= n8) continue;
@@ -171,7 +175,7 @@ __global__ __launch_bounds__(kNormThreads) void k_combine_add_rms_norm(
   for (int i = 0; i < kNormThreads / 64; ++i) tot += s_part[i];
   const float r = 1.0f / sqrtf(tot / (float)H + eps);
 #pragma unroll
-  for (int q = 0; q < kNormChunks; ++q) {
+  for (int q = 0; q < NQ; ++q) {
     const int c8 = tid + kNormThreads * q;
     if (c8 >= n8) continue;
     const uint32_t x4[4] = {xv[q].x, xv[q].y, xv[q].z, xv[q].w};
@@ -197,8 +201,17 @@ hipError_t launch_combine_add_rms_norm(const uint16_t* dn, const int64_t* idx, c
                                        int topk, int E, int H, float eps, hipStream_t s) {
   if (M == 0) return hipSuccess;
   if (topk <= 0 || topk > 8 || H % 8 != 0 || H > kNormThreads * kNormChunks * 8) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_combine_add_rms_norm, dim3((unsigned)M), dim3(kNormThreads), 0, s, dn, idx, tw, h, w, out,
-                     h_out, y, topk, E, H, eps);
+  const dim3 grid((unsigned)M), block(kNormThreads);
+#define W4A16_CAN(NQ_)                                                                                             \
+  hipLaunchKernelGGL(k_combine_add_rms_norm<NQ_>, grid, block, 0, s, dn, idx, tw, h, w, out, h_out, y, topk, E, H, \
+                     eps)
+  switch ((H / 8 + kNormThreads - 1) / kNormThreads) {
+    case 1: W4A16_CAN(1); break;
+    case 2: W4A16_CAN(2); break;
+    case 3: W4A16_CAN(3); break;
+    default: W4A16_CAN(4); break;
+  }
+#undef W4A16_CAN
   return hipGetLastError();
 }
 
@@ -207,8 +220,15 @@ hipError_t launch_add_rms_norm(const uint16_t* h, const uint16_t* delta, const u
                                hipStream_t s) {
   if (M == 0) return hipSuccess;
   if (H % 8 != 0 || H > kNormThreads * kNormChunks * 8) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_add_rms_norm, dim3((unsigned)M), dim3(kNormThreads), 0, s, h, delta, w,
-                     h_out, y, H, eps);
+  const dim3 grid((unsigned)M), block(kNormThreads);
+#define W4A16_AN(NQ_) hipLaunchKernelGGL(k_add_rms_norm<NQ_>, grid, block, 0, s, h, delta, w, h_out, y, H, eps)
+  switch ((H / 8 + kNormThreads - 1) / kNormThreads) {
+    case 1: W4A16_AN(1); break;
+    case 2: W4A16_AN(2); break;
+    case 3: W4A16_AN(3); break;
+    default: W4A16_AN(4); break;
+  }
+#undef W4A16_AN
   return hipGetLastError();
 }
 

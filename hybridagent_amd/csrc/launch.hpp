@@ -275,10 +275,16 @@ hipError_t launch_topk_sort_with_linear(const float* partial, int ksplit, const 
 hipError_t launch_ffn_pre(const uint16_t* attn, const uint16_t* res, const uint16_t* w_pa,
                           const uint16_t* w_pf, const uint16_t* w_pf2, uint16_t* res_out, uint16_t* h_ff,
                           uint16_t* h2_in, int64_t M, int H, float eps, hipStream_t s);
-hipError_t launch_ffn_post(const uint16_t* mlp, const uint16_t* moe, const uint16_t* res,
-                           const uint16_t* w1, const uint16_t* w2, const uint16_t* w3,
-                           const uint16_t* layer_scalar, uint16_t* out, int64_t M, int H, float eps,
-                           hipStream_t s);
+struct FfnPostCall {
+  const uint16_t *mlp, *res, *w1, *w2, *w3, *layer_scalar;
+  uint16_t* out;
+  float eps;
+};
+// moe: the experts' output rows, or (idx non-null, topk as ffn_post_combines
+// says) their rows t * topk + j, which the launch combines with tw first
+bool ffn_post_combines(int64_t topk);
+hipError_t launch_ffn_post(const FfnPostCall& c, const uint16_t* moe, const int64_t* idx, const float* tw, int topk,
+                           int E, int64_t M, int H, hipStream_t s);
 // BF16 experts: grid (column tile, active slot), max_slots <= 65535
 hipError_t launch_bf16_experts(int mode, Bf16ExpertArgs a, int max_slots, hipStream_t s);
 // Linear4Bit at prefill sizes (kernels_linear_w4.hip): K a multiple of 32

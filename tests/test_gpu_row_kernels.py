@@ -1,0 +1,49 @@
+"""The row kernels built per 16-byte chunks of a thread (H <= 2048, 4096, 6144, 8192)
+and the FFN block's last launch with the combine inside: a token's row equals,
+bit for bit, the same token's in calls of four (32 routed rows: the fused down +
+combine, then the block's last launch on its output), at each chunk count, and
+at top_k = 9, which combines in a launch of its own.  The norms against torch."""
+import math
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+from hybridagent_amd import _lib, synth
+
+pytestmark = pytest.mark.gpu
+
+# rows of one chunk and less, edges of one, two, three and four chunks per thread
+WIDTHS = [256, 2048, 2080, 2816, 4096, 4128, 6144, 8192]
+
+
+@pytest.mark.parametrize("H", WIDTHS)
+@pytest.mark.parametrize("k", [8, 9])
+def test_ffn_post_combines_bit_identical(H, k):
+    dev = torch.device("cuda:0")
+    E, I, Im, G, M = 16, 64, 96, 32, 12
+    g = torch.Generator().manual_seed(H + k)
+    nrm = lambda: (1 + 0.1 * torch.randn(H, generator=g)).to(torch.bfloat16).to(dev)
+    lin = lambda o, i: (torch.randn(o, i, generator=g) / math.sqrt(i)).to(torch.bfloat16).to(dev)
+    w = synth.moe_weights(E, H, I, G, seed=3, device=dev)
+    rw = synth.router_weights(E, H, seed=4, device=dev)
+    res, att = synth.activations(M, H, 5, dev), synth.activations(M, H, 6, dev)
+    tail = (nrm(), nrm(), lin(Im, H), lin(Im, H), lin(H, Im), nrm(), nrm(), H ** -0.5, rw.proj, rw.per_expert_scale,
+            nrm(), w.gate_up_packed, w.gate_up_scale, w.down_packed, w.down_scale, nrm(), nrm(),
+            torch.full((1,), 0.5, dtype=torch.bfloat16, device=dev), 1e-6, k, G)
+    y = _lib.ffn_block(res, att, *tail)
+    step = 4 if k == 8 else 3
+    for m in range(0, M, step):
+        assert torch.equal(_lib.ffn_block(res[m:m + step], att[m:m + step], *tail), y[m:m + step]), f"rows {m}.."
+
+
+@pytest.mark.parametrize("H", WIDTHS)
+def test_norms(H):
+    dev = torch.device("cuda:0")
+    x, d = synth.activations(5, H, 7, dev), synth.activations(5, H, 8, dev)
+    w = (1 + 0.1 * torch.randn(H, generator=torch.Generator().manual_seed(9))).to(torch.bfloat16).to(dev)
+    h, y = _lib.add_rms_norm(x, w, 1e-6, d)
+    assert torch.equal(h, x + d)
+    ref = F.rms_norm(h.double(), (H,), w.double(), 1e-6)
+    # one rounding to bf16 (half a unit: 2^-8), and fp32 sums of H squares
+    assert ((y.double() - ref).abs() <= 2.0 ** -8 * ref.abs() * (1 + 2.0 ** -7)).all()
