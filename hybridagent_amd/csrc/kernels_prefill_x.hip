@@ -1114,15 +1114,12 @@ hipError_t launch_tile_prefill(int mode, const int32_t* packed, int E, int H, in
 // persistent grid: the workgroups that fit on the device at once (a multiple
 // of the 8 XCDs), at most one per item
 int prefill_grid_size(const void* kern, int threads, size_t lds, int max_items) {
-  int dev = 0, cus = 256, per_cu = 1;
-  hipDeviceProp_t p;
-  if (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&p, dev) == hipSuccess &&
-      p.multiProcessorCount > 0)
-    cus = p.multiProcessorCount;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, threads, lds) != hipSuccess ||
-      per_cu <= 0)
+  int per_cu = 1;
+  // more than half of a CU's LDS: one workgroup, nothing to ask the runtime
+  if (2 * lds <= 160 * 1024 &&
+      (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, threads, lds) != hipSuccess || per_cu <= 0))
     per_cu = 1;
-  int g = cus * per_cu;
+  int g = device_cus() * per_cu;
   if (max_items < g) g = max_items;
   return ((g + 7) / 8) * 8;
 }

@@ -328,6 +328,8 @@ hipError_t launch_prefill_x(int mode, PrefillArgs a, int max_mtiles, hipStream_t
 size_t prefill_tiled_bytes_per_expert(int mode, int64_t H, int64_t I);
 hipError_t launch_tile_prefill(int mode, const int32_t* packed, int E, int H, int I, int32_t* tiled,
                                hipStream_t s);
+// CUs of the current device
+int device_cus();
 // persistent prefill grid: the workgroups that fit at once (a multiple of the
 // 8 XCDs), at most max_items
 int prefill_grid_size(const void* kern, int threads, size_t lds, int max_items);
