@@ -18,16 +18,15 @@
 //
 // The small tails (most of them are whole experts of few rows) give a stage
 // little MFMA work, so what a stage costs whatever its rows decides.
-//  - Tails of 33..64 rows, and on the packed weights of 1..32, run as tail
-//    items (px_run_t): stages of 128 k, the item's scales read once as one
-//    contiguous block.  128 experts of 64 rows at the Gemma shape, G = 128,
-//    tiled: gate_up 144 -> 116 us, down 90 -> 76 us; packed layers of 257
-//    tokens x top-8 at G = 32 / 128 322 -> 162 / 173 -> 157 us (with a 16-byte
-//    scale chunk per row and stage the 768 rows of a three-n-tile stage
-//    touched more cache lines than an XCD's L2 holds).
-//  - On the tiled weights a tail of at most 32 rows is a wide item of three
-//    n-tiles (px_run_w): one stage's cost for three n-tiles' weights.  257
-//    tokens: 140-146 us, as tail items 154 us.
+//  - They run as tail items (px_run_t): stages of 128 k, the item's scales
+//    read once as one contiguous block.  128 experts of 64 rows at the Gemma
+//    shape, G = 128, tiled: gate_up 144 -> 116 us, down 90 -> 76 us; packed
+//    layers of 257 tokens x top-8 at G = 32 / 128 322 -> 162 / 173 -> 157 us
+//    (with a 16-byte scale chunk per row and stage the 768 rows of a
+//    three-n-tile stage touched more cache lines than an XCD's L2 holds).
+//  - On the tiled weights, where nearly all m-tiles are tails of at most 32
+//    rows, each is a wide item of three n-tiles (px_run_w): one stage's cost
+//    for three n-tiles' weights.
 // Each output is the one-n-tile item's bit for bit.
 //
 // Per 64-wide k stage, all by direct global -> LDS loads of 16 bytes per
@@ -133,31 +132,35 @@ struct PxItem {
   int nt, e, seg0, nrows, mb, nb;
 };
 
-// Item `item` of a queue whose m-tiles are tile list entries x0, x0 + xs, ...:
-// m-tiles [t0, t1) of the queue (with tiled weights the tails of at most
-// kPrefillTinyRows rows, else none) have n_wide items of kPxWide n-tiles each
-// (n-tiles past the matrix compute on its last rows and store nothing), the
-// others n_nt items of one n-tile.
-__device__ __forceinline__ PxItem px_item_info(const PrefillArgs& a, int x0, int xs, int t0, int t1, int n_wide,
-                                               int item) {
+// Item `item` of a queue of n_local m-tiles, tile list entries x0, x0 + xs,
+// ...; [t0, t1) are the tails of at most kPrefillTinyRows rows.  With n_wide
+// > 0 these are wide items, n_wide of kPxWide n-tiles each (n-tiles past the
+// matrix compute on its last rows and store nothing), where they stand in the
+// list: a wide item is longer than the tails after it.  Else every m-tile has
+// n_nt items, the tails [t0, t1) last: they are the shortest.
+__device__ __forceinline__ PxItem px_item_info(const PrefillArgs& a, int x0, int xs, int n_local, int t0, int t1,
+                                               int n_wide, int item) {
   PxItem it;
-  const int i0 = t0 * a.n_nt, i1 = i0 + (t1 - t0) * n_wide;
   int lm;
   it.nb = 1;
-  if (item < i0) {
+  const int i0 = t0 * a.n_nt, i1 = i0 + (t1 - t0) * n_wide;
+  if (n_wide > 0 && item >= i0) {
+    if (item < i1) {
+      const int j = item - i0;
+      const int q = j / n_wide;
+      lm = t0 + q;
+      it.nt = kPxWide * (j - q * n_wide);
+      it.nb = kPxWide;
+    } else {
+      const int j = item - i1;
+      const int q = j / a.n_nt;
+      lm = t1 + q;
+      it.nt = j - q * a.n_nt;
+    }
+  } else {
     lm = item / a.n_nt;
     it.nt = item - lm * a.n_nt;
-  } else if (item < i1) {
-    const int j = item - i0;
-    const int q = j / n_wide;
-    lm = t0 + q;
-    it.nt = kPxWide * (j - q * n_wide);
-    it.nb = kPxWide;
-  } else {
-    const int j = item - i1;
-    const int q = j / a.n_nt;
-    lm = t1 + q;
-    it.nt = j - q * a.n_nt;
+    if (n_wide == 0 && lm >= t0) lm = lm - t0 < n_local - t1 ? lm - t0 + t1 : lm - (n_local - t1);
   }
   const int tile = ld_uniform(a.tiles, x0 + xs * lm);
   it.e = tile >> 16;
@@ -168,11 +171,9 @@ __device__ __forceinline__ PxItem px_item_info(const PrefillArgs& a, int x0, int
 }
 
 // whether a one-n-tile item runs as a tail item (px_run_t): one or two
-// m-blocks; with tiled weights two (one m-block is a wide item there)
-template <bool TILED>
+// m-blocks
 __device__ __forceinline__ bool px_is_tail(const PrefillArgs& a, const PxItem& it) {
-  if (it.mb == 2) return a.tail_s1[1] >= 0;
-  return !TILED && it.mb == 1 && a.tail_s1[0] >= 0;
+  return it.mb <= kPxTailMaxBlocks && a.tail_s1[it.mb == 2 ? 1 : 0] >= 0;
 }
 
 // A lane's load sources for one item; na = the wavefront's A loads per
@@ -468,8 +469,8 @@ __device__ __forceinline__ int px_issue_first(const PrefillArgs& a, const PxItem
     for (int p = 0; p < 4; ++p) px_issue_w(a, L, smem, 1, 1, p);
     return L.n;
   }
-  if (px_is_tail<TILED>(a, it)) {
-    if (!TILED && it.mb == 1) return px_issue_first_t<MODE, TILED, 1>(a, it, smem);
+  if (px_is_tail(a, it)) {
+    if (it.mb == 1) return px_issue_first_t<MODE, TILED, 1>(a, it, smem);
     return px_issue_first_t<MODE, TILED, 2>(a, it, smem);
   }
   const PxLoads L = px_loads<MODE, TILED>(a, it, smem);
@@ -956,9 +957,8 @@ __device__ __forceinline__ int px_dispatch(const PrefillArgs& a, unsigned char* 
     if (it.nb > 1) return px_run_w<MODE, TILED>(a, smem, it, nx, has_next, n_inflight, fetch_q);
   // gate_up's half n-tile: eight wavefronts on four wavefronts' columns
   const bool half = MODE == kModeGateUp && a.I - 128 * it.nt == 64;
-  if (px_is_tail<TILED>(a, it)) {
-    if constexpr (!TILED)
-      if (it.mb == 1) return px_run_t<MODE, TILED, 1>(a, smem, it, nx, has_next, fetch_q);
+  if (px_is_tail(a, it)) {
+    if (it.mb == 1) return px_run_t<MODE, TILED, 1>(a, smem, it, nx, has_next, fetch_q);
     if constexpr (MODE == kModeGateUp)
       if (half) return px_run_t<MODE, TILED, 1, 2>(a, smem, it, nx, has_next, fetch_q);
     return px_run_t<MODE, TILED, 2>(a, smem, it, nx, has_next, fetch_q);
@@ -1005,9 +1005,7 @@ __global__ __launch_bounds__(kPxThreads) __attribute__((amdgpu_waves_per_eu(2, 2
 void k_prefill_x(PrefillArgs a) {
   extern __shared__ __align__(16) unsigned char smem[];
   const int ntiles = ld_uniform(a.counters, 1);
-  // the tails that run as wide items (tiled weights)
-  const int tiny0 = TILED ? ld_uniform(a.counters, 2) : 0;
-  const int tiny1 = TILED ? ld_uniform(a.counters, 3) : 0;
+  const int tiny0 = ld_uniform(a.counters, 2), tiny1 = ld_uniform(a.counters, 3);  // the smallest tails
   constexpr bool kChip = MODE == kModeGateUp;  // one queue for the chip
   const int x0 = kChip ? 0 : (int)(blockIdx.x & 7);
   const int xs = kChip ? 1 : 8;
@@ -1015,8 +1013,14 @@ void k_prefill_x(PrefillArgs a) {
   // the queue's m-tiles before list entry b
   auto local = [&](int b) { return kChip ? b : (b > x0 ? (b - x0 + 7) >> 3 : 0); };
   const int t0 = local(tiny0), t1 = local(tiny1);
-  const int n_wide = (a.n_nt + kPxWide - 1) / kPxWide;
-  const int it_end = (n_local - (t1 - t0)) * a.n_nt + (t1 - t0) * n_wide;
+  // Wide items where the m-tiles are smallest tails but for one in fifty: of
+  // like length, they go round once.  Among other items their own length (two
+  // to three times a tail's) shows at the end: at the Gemma shape, tiled, G =
+  // 128 / 32, as wide / tail items, 257 tokens of flat routing 139/155,
+  // 160/163 us; 400 tokens 167/158, 191/166; 257 tokens skewed 182/173,
+  // 206/178; 1536 tokens skewed 311/280, 325/283.
+  const int n_wide = TILED && 50 * (tiny1 - tiny0) >= 49 * ntiles ? (a.n_nt + kPxWide - 1) / kPxWide : 0;
+  const int it_end = (n_local - (t1 - t0)) * a.n_nt + (t1 - t0) * (n_wide > 0 ? n_wide : a.n_nt);
   const int P = kChip ? (int)gridDim.x : (int)(gridDim.x >> 3);
   int* const queue = a.queues != nullptr ? a.queues + x0 : nullptr;
   // the last workgroup to leave resets the counters for the next launch
@@ -1034,7 +1038,7 @@ void k_prefill_x(PrefillArgs a) {
     leave();
     return;
   }
-  PxItem cur = px_item_info(a, x0, xs, t0, t1, n_wide, item);
+  PxItem cur = px_item_info(a, x0, xs, n_local, t0, t1, n_wide, item);
   if (MODE == kModeGateUp) {
     // the first item's gathered rows into the table (nothing else in flight)
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1048,7 +1052,7 @@ void k_prefill_x(PrefillArgs a) {
   int nitem = item + P;
   for (;;) {
     const bool has_next = nitem < it_end;
-    const PxItem nxt = has_next ? px_item_info(a, x0, xs, t0, t1, n_wide, nitem) : cur;
+    const PxItem nxt = has_next ? px_item_info(a, x0, xs, n_local, t0, t1, n_wide, nitem) : cur;
     // with a next item, take the index of the one after it during this item
     n_inflight = px_dispatch<MODE, TILED>(a, smem, cur, nxt, has_next, n_inflight, has_next ? queue : nullptr);
     if (!has_next) break;

@@ -46,3 +46,22 @@ def test_tail_rows_bit_identical(h, i, G, tiled):
     ref = oracle.moe_forward(np_(x[pick]), idx[pick][:, None].numpy(), np_(w[pick]), wts.gate_up_packed.cpu().numpy(),
                              bits(wts.gate_up_scale), wts.down_packed.cpu().numpy(), bits(wts.down_scale), G)
     assert margin(f"prefill tails h={h} i={i} G={G}", oracle.max_abs_rel(np_(a[pick]), ref)) <= TOL
+
+
+@pytest.mark.parametrize("extra", [0, 40])
+@pytest.mark.parametrize("h,i,G", [(384, 320, 32), (2816, 704, 128)])
+def test_wide_items_only_among_small_tails(h, i, G, extra):
+    # every expert a tail of at most 32 rows: the tiled weights' wide items; with one expert of 60 rows: tail items
+    dev = torch.device("cuda:0")
+    e, r = 18, 20
+    wts = synth.moe_weights(e, h, i, G, seed=44, device=dev)
+    gpu = [wts.gate_up_packed, wts.gate_up_scale, wts.down_packed, wts.down_scale]
+    tiles = _lib.tile_experts(*gpu, G)
+    idx = torch.cat([torch.arange(e).repeat(r), torch.zeros(extra, dtype=torch.long)])[:, None].to(dev)
+    x = synth.activations(idx.shape[0], h, seed=45, device=dev)
+    w = torch.ones(idx.shape[0], 1, device=dev)
+    print(f"wide h={h} i={i} G={G} extra={extra}", flush=True)
+    a = _lib.moe_forward(x, idx, w, *gpu, G, tiles=tiles)
+    assert torch.equal(a, _lib.moe_forward(x, idx, w, *gpu, G, tiles=None))
+    if extra:
+        assert torch.equal(a[:e * r], _lib.moe_forward(x[:e * r], idx[:e * r], w[:e * r], *gpu, G, tiles=tiles))
