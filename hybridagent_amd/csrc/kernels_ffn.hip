@@ -21,6 +21,7 @@
 // order), so a row's result does not depend on the batch around it.
 #include "common.hpp"
 #include "launch.hpp"
+#include "linear_bf16.hpp"
 
 namespace w4a16 {
 
@@ -106,7 +107,7 @@ __device__ __forceinline__ void norm8(const Row8& x, float rstd, const Row8& w, 
 
 }  // namespace
 
-template <int NQ>
+template <int NQ, bool FRAG>
 __global__ __launch_bounds__(kFfnThreads) void k_ffn_pre(
     const uint16_t* __restrict__ attn, const uint16_t* __restrict__ res, const uint16_t* __restrict__ w_pa,
     const uint16_t* __restrict__ w_pf, const uint16_t* __restrict__ w_pf2, uint16_t* __restrict__ res_out,
@@ -155,7 +156,10 @@ __global__ __launch_bounds__(kFfnThreads) void k_ffn_pre(
     if (c8 >= n8) continue;
     float o[8];
     norm8(r[q], rsr, conv8(wf[q]), o);
-    store8(h_ff + off, c8, o);
+    if (FRAG)
+      store8(h_ff + frag_index(blockIdx.x, 8 * c8, H), 0, o);
+    else
+      store8(h_ff + off, c8, o);
     norm8(r[q], rsr, conv8(wf2[q]), o);
     store8(h2_in + off, c8, o);
   }
@@ -267,12 +271,19 @@ __global__ __launch_bounds__(kFfnThreads) void k_ffn_post(
 
 hipError_t launch_ffn_pre(const uint16_t* attn, const uint16_t* res, const uint16_t* w_pa,
                           const uint16_t* w_pf, const uint16_t* w_pf2, uint16_t* res_out, uint16_t* h_ff,
-                          uint16_t* h2_in, int64_t M, int H, float eps, hipStream_t s) {
+                          uint16_t* h2_in, int64_t M, int H, float eps, bool frag, hipStream_t s) {
   if (M == 0) return hipSuccess;
-  if (H % 8 != 0 || H > kFfnThreads * kFfnChunks * 8) return hipErrorInvalidValue;
+  if (H % 8 != 0 || H > kFfnThreads * kFfnChunks * 8 || (frag && H % 32 != 0)) return hipErrorInvalidValue;
   const dim3 grid((unsigned)M), block(kFfnThreads);
-#define W4A16_PRE(NQ_) \
-  hipLaunchKernelGGL(k_ffn_pre<NQ_>, grid, block, 0, s, attn, res, w_pa, w_pf, w_pf2, res_out, h_ff, h2_in, H, eps)
+#define W4A16_PRE(NQ_)                                                                                              \
+  do {                                                                                                              \
+    if (frag)                                                                                                       \
+      hipLaunchKernelGGL((k_ffn_pre<NQ_, true>), grid, block, 0, s, attn, res, w_pa, w_pf, w_pf2, res_out, h_ff,    \
+                         h2_in, H, eps);                                                                            \
+    else                                                                                                            \
+      hipLaunchKernelGGL((k_ffn_pre<NQ_, false>), grid, block, 0, s, attn, res, w_pa, w_pf, w_pf2, res_out, h_ff,   \
+                         h2_in, H, eps);                                                                            \
+  } while (0)
   switch ((H / 8 + kFfnThreads - 1) / kFfnThreads) {
     case 1: W4A16_PRE(1); break;
     case 2: W4A16_PRE(2); break;

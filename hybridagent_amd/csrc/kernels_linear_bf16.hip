@@ -15,6 +15,7 @@
 //   kLinGateUp    bf16(bf16(gelu_tanh(bf16(acc_gate))) * bf16(acc_up))
 //                 gate rows from W, up rows from W2              shared MLP gate/up
 //   kLinPlain     bf16(acc)                                      shared MLP down
+//   kLinGateUpFrag, kLinPlainFrag  the same two on fragment-order rows
 // Every rounding point is one of the torch bf16 module's (F.linear rounds its
 // output, the activation and the product round theirs).
 #include "linear_bf16.hpp"
@@ -42,6 +43,8 @@ hipError_t launch_linear_bf16(int epi, const uint16_t* x, const uint16_t* W, con
       case kLinGelu: hipLaunchKernelGGL((k_linear_bf16<MT_, kLinGelu>), grid, block, 0, s, a); break; \
       case kLinResidual: hipLaunchKernelGGL((k_linear_bf16<MT_, kLinResidual>), grid, block, 0, s, a); break; \
       case kLinGateUp: hipLaunchKernelGGL((k_linear_bf16<MT_, kLinGateUp>), grid, block, 0, s, a); break; \
+      case kLinGateUpFrag: hipLaunchKernelGGL((k_linear_bf16<MT_, kLinGateUpFrag>), grid, block, 0, s, a); break; \
+      case kLinPlainFrag: hipLaunchKernelGGL((k_linear_bf16<MT_, kLinPlainFrag>), grid, block, 0, s, a); break; \
       default: hipLaunchKernelGGL((k_linear_bf16<MT_, kLinPlain>), grid, block, 0, s, a); break; \
     }                                                                                      \
   } while (0)

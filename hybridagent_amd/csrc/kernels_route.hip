@@ -848,7 +848,7 @@ hipError_t launch_topk_sort(const float* partial, int ksplit, const uint16_t* pe
 static_assert(kFusedLogitsThreads == kLinThreads && 64 * kSmallSortWaves == kLinThreads,
               "one workgroup size for the fused bodies");
 
-template <int MT>
+template <int MT, int EPI>
 __global__ __launch_bounds__(kLinThreads) void k_router_logits_with_linear(RouterNormLogitsArgs ra, int rgx,
                                                                          int rblocks, LinArgs la, int lgx) {
   const int b = blockIdx.x;
@@ -857,7 +857,7 @@ __global__ __launch_bounds__(kLinThreads) void k_router_logits_with_linear(Route
     return;
   }
   const int l = b - rblocks;
-  linear_bf16_block<MT, kLinGateUp>(la, l % lgx, l / lgx);
+  linear_bf16_block<MT, EPI>(la, l % lgx, l / lgx);
 }
 
 template <int PER>
@@ -873,24 +873,28 @@ __global__ __launch_bounds__(kLinThreads) void k_topk_sort_with_linear(TopkSortA
 hipError_t launch_router_norm_logits_with_linear(const uint16_t* h, const uint16_t* scale, float scalar_root,
                                                  float eps, const uint16_t* proj, float* partial, int M, int H,
                                                  int E, int ksplit, const LinearCall& lin, hipStream_t s) {
-  if (M == 0 || lin.M != M || lin.epi != kLinGateUp || lin.K % 32 != 0 || lin.K <= 0 || lin.N <= 0)
+  if (M == 0 || lin.M != M || !lin_gate_up(lin.epi) || lin.K % 32 != 0 || lin.K <= 0 || lin.N <= 0)
     return hipErrorNotSupported;
   const int nchunks = H >> 5;
   const int per = (nchunks + ksplit - 1) / ksplit;
   if (per > kFusedLogitsMaxSteps) return hipErrorNotSupported;
   const int mt = lin_row_tiles(lin.M);
-  if (mt > 2) return hipErrorNotSupported;
+  if (mt > 2 || (mt == 1 && lin.epi == kLinGateUpFrag)) return hipErrorNotSupported;
   const RouterNormLogitsArgs ra{h, scale, scalar_root, eps, proj, partial, M, H, E, per};
   const int rgx = (M + 15) / 16, rblocks = rgx * ksplit;
   const LinArgs la = lin_args(lin.epi, lin.x, lin.W, lin.W2, lin.bias, lin.res, lin.out, lin.M, lin.N, lin.K);
   const int lgx = lin_grid_x(lin.epi, lin.N);
   const int64_t blocks = rblocks + (int64_t)lgx * lin_grid_y(lin.M);
+#define W4A16_RL(MT_, EPI_)                                                                                     \
+  hipLaunchKernelGGL((k_router_logits_with_linear<MT_, EPI_>), dim3((unsigned)blocks), dim3(kLinThreads), 0, s, ra, \
+                     rgx, rblocks, la, lgx)
   if (mt == 1)
-    hipLaunchKernelGGL(k_router_logits_with_linear<1>, dim3((unsigned)blocks), dim3(kLinThreads), 0, s, ra, rgx,
-                       rblocks, la, lgx);
+    W4A16_RL(1, kLinGateUp);
+  else if (lin.epi == kLinGateUp)
+    W4A16_RL(2, kLinGateUp);
   else
-    hipLaunchKernelGGL(k_router_logits_with_linear<2>, dim3((unsigned)blocks), dim3(kLinThreads), 0, s, ra, rgx,
-                       rblocks, la, lgx);
+    W4A16_RL(2, kLinGateUpFrag);
+#undef W4A16_RL
   return hipGetLastError();
 }
 

@@ -242,7 +242,16 @@ hipError_t launch_layer_norm(const uint16_t* x, const uint16_t* w, const uint16_
 //   kLinGateUp    out = bf16(bf16(gelu_tanh(bf16(x W^T))) * bf16(x W2^T))
 //   kLinPlain     out = bf16(x W^T)
 // M rows in tiles of up to 64 (ceil(M / 64) <= 65535).
-enum LinearEpilogue { kLinGelu = 0, kLinResidual = 1, kLinGateUp = 2, kLinPlain = 3 };
+//   kLinGateUpFrag, kLinPlainFrag: kLinGateUp with x and out, kLinPlain with
+//   x in fragment order (linear_bf16.hpp)
+enum LinearEpilogue {
+  kLinGelu = 0,
+  kLinResidual = 1,
+  kLinGateUp = 2,
+  kLinPlain = 3,
+  kLinGateUpFrag = 4,
+  kLinPlainFrag = 5
+};
 hipError_t launch_linear_bf16(int epi, const uint16_t* x, const uint16_t* W, const uint16_t* W2,
                               const uint16_t* bias, const uint16_t* res, uint16_t* out, int64_t M, int N,
                               int K, hipStream_t s);
@@ -255,10 +264,11 @@ struct LinearCall {
   int64_t M;
   int N, K;
 };
-// launch_router_norm_logits with a kLinGateUp linear of at most 32 rows in the
-// same launch; launch_topk_sort (one top-k round, E <= 128) with a kLinPlain
-// linear of at most 16 rows.  hipErrorNotSupported (nothing launched) where
-// the shapes need separate launches.
+// launch_router_norm_logits with a gate/up linear of at most 32 rows (in
+// fragment order: 17..32) in the same launch; launch_topk_sort (one top-k
+// round, E <= 128) with a kLinPlain linear of at most 16 rows.
+// hipErrorNotSupported (nothing launched) where the shapes need separate
+// launches.
 hipError_t launch_router_norm_logits_with_linear(const uint16_t* h, const uint16_t* scale, float scalar_root,
                                                  float eps, const uint16_t* proj, float* partial, int M, int H,
                                                  int E, int ksplit, const LinearCall& lin, hipStream_t s);
@@ -268,13 +278,14 @@ hipError_t launch_topk_sort_with_linear(const float* partial, int ksplit, const 
                                         int BM, int slot_rows, const LinearCall& lin, hipStream_t s);
 // FFN block row kernels (kernels_ffn.hip), one workgroup per row, H % 8 == 0,
 // H <= 8192:
+//   (frag: h_ff in the bf16 linears' fragment order, H % 32 == 0)
 //   pre : h = rms(attn) * w_pa; res_out = bf16(res + h);
 //         h_ff = rms(res_out) * w_pf; h2_in = rms(res_out) * w_pf2
 //   post: h1 = rms(mlp) * w1; h2 = rms(moe) * w2; c = rms(bf16(h1 + h2)) * w3;
 //         out = bf16(bf16(res + c) * layer_scalar)
 hipError_t launch_ffn_pre(const uint16_t* attn, const uint16_t* res, const uint16_t* w_pa,
                           const uint16_t* w_pf, const uint16_t* w_pf2, uint16_t* res_out, uint16_t* h_ff,
-                          uint16_t* h2_in, int64_t M, int H, float eps, hipStream_t s);
+                          uint16_t* h2_in, int64_t M, int H, float eps, bool frag, hipStream_t s);
 struct FfnPostCall {
   const uint16_t *mlp, *res, *w1, *w2, *w3, *layer_scalar;
   uint16_t* out;

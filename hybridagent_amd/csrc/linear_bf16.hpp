@@ -5,8 +5,9 @@
 // columns and the same 8 up columns) for up to 16 * MT rows.
 //
 // Fragment order (the HybridLink chain's activations, kLinGelu's input and
-// output, kLinResidual's input): rows padded to a multiple of 16, element
-// (m, k) of a [Mp, K] matrix at
+// output, kLinResidual's input; the FFN block's from 17 rows on,
+// kLinGateUpFrag's input and output, kLinPlainFrag's input): rows padded to a
+// multiple of 16, element (m, k) of a [Mp, K] matrix at
 //   ((m / 16) * (K / 32) + k / 32) * 512 + ((k % 32) / 8) * 128 + (m % 16) * 8 + k % 8,
 // so the 16 rows x 32 k of one MFMA step's A operand are one contiguous KiB
 // (lane l's 16 bytes at 16 l) instead of 16 rows x 64 bytes: the activation
@@ -40,7 +41,8 @@ inline LinArgs lin_args(int, const uint16_t* x, const uint16_t* W, const uint16_
   const int nsteps = K >> 5;
   return LinArgs{x, W, W2, bias, res, out, (int)M, N, K, (nsteps + kLinWaves - 1) / kLinWaves};
 }
-inline int lin_grid_x(int epi, int N) { return (N + (epi == kLinGateUp ? 8 : 16) - 1) / (epi == kLinGateUp ? 8 : 16); }
+constexpr bool lin_gate_up(int epi) { return epi == kLinGateUp || epi == kLinGateUpFrag; }
+inline int lin_grid_x(int epi, int N) { return (N + (lin_gate_up(epi) ? 8 : 16) - 1) / (lin_gate_up(epi) ? 8 : 16); }
 inline int64_t lin_grid_y(int64_t M) { return (M + 16 * lin_row_tiles(M) - 1) / (16 * lin_row_tiles(M)); }
 
 // element (m, k) of a fragment-order matrix with K columns
@@ -48,13 +50,15 @@ __host__ __device__ inline int64_t frag_index(int64_t m, int k, int K) {
   return ((m >> 4) * (K >> 5) + (k >> 5)) * 512 + ((k & 31) >> 3) * 128 + (m & 15) * 8 + (k & 7);
 }
 // the epilogues whose input (XF) and output (OF) are in fragment order
-constexpr bool lin_x_frag(int epi) { return epi == kLinGelu || epi == kLinResidual; }
-constexpr bool lin_out_frag(int epi) { return epi == kLinGelu; }
+constexpr bool lin_x_frag(int epi) {
+  return epi == kLinGelu || epi == kLinResidual || epi == kLinGateUpFrag || epi == kLinPlainFrag;
+}
+constexpr bool lin_out_frag(int epi) { return epi == kLinGelu || epi == kLinGateUpFrag; }
 
 template <int MT, int EPI>
 __device__ __forceinline__ void linear_bf16_block(const LinArgs& a, int bx, int by) {
   __shared__ f32x4_t red[kLinWaves][MT][64];
-  constexpr bool GU = EPI == kLinGateUp;
+  constexpr bool GU = lin_gate_up(EPI);
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int j = lane & 15, kb = lane >> 4;
@@ -125,7 +129,8 @@ __device__ __forceinline__ void linear_bf16_block(const LinArgs& a, int bx, int 
           if (m < a.M) {
             const float gate = round_bf16(t[q]);
             const float act = round_bf16(gelu_tanh_f32(gate));
-            a.out[(int64_t)m * a.N + n] = f32_to_bf16_bits(act * round_bf16(up[q]));
+            a.out[lin_out_frag(EPI) ? frag_index(m, n, a.N) : (int64_t)m * a.N + n] =
+                f32_to_bf16_bits(act * round_bf16(up[q]));
           }
         }
       }
@@ -138,7 +143,7 @@ __device__ __forceinline__ void linear_bf16_block(const LinArgs& a, int bx, int 
           const int m = m0 + 16 * i + 4 * kb + q;
           if (m < a.M) {
             float o;
-            if (EPI == kLinPlain) {
+            if (EPI == kLinPlain || EPI == kLinPlainFrag) {
               o = t[q];
             } else {
               const float v = round_bf16(t[q] + bn);

@@ -37,6 +37,29 @@ def test_ffn_post_combines_bit_identical(H, k):
         assert torch.equal(_lib.ffn_block(res[m:m + step], att[m:m + step], *tail), y[m:m + step]), f"rows {m}.."
 
 
+# The shared MLP's rows in fragment order from 17 rows on (row tiles of 2 and 4,
+# partial last tiles), and row-major where they don't fit (top_k 1;
+# 2 at the wide Im): every row as in calls of 16 rows, which never use that order.
+@pytest.mark.parametrize("M", [17, 31, 32, 33, 48, 63, 64])
+@pytest.mark.parametrize("H,Im", [(256, 96), (2816, 2112), (512, 1056)])
+@pytest.mark.parametrize("k", [1, 2, 8])
+def test_ffn_fragment_rows_bit_identical(M, H, Im, k):
+    dev = torch.device("cuda:0")
+    E, I, G = 16, 64, 32
+    g = torch.Generator().manual_seed(M + H + k)
+    nrm = lambda: (1 + 0.1 * torch.randn(H, generator=g)).to(torch.bfloat16).to(dev)
+    lin = lambda o, i: (torch.randn(o, i, generator=g) / math.sqrt(i)).to(torch.bfloat16).to(dev)
+    w = synth.moe_weights(E, H, I, G, seed=3, device=dev)
+    rw = synth.router_weights(E, H, seed=4, device=dev)
+    res, att = synth.activations(M, H, 5, dev), synth.activations(M, H, 6, dev)
+    tail = (nrm(), nrm(), lin(Im, H), lin(Im, H), lin(H, Im), nrm(), nrm(), H ** -0.5, rw.proj, rw.per_expert_scale,
+            nrm(), w.gate_up_packed, w.gate_up_scale, w.down_packed, w.down_scale, nrm(), nrm(),
+            torch.full((1,), 0.5, dtype=torch.bfloat16, device=dev), 1e-6, k, G)
+    y = _lib.ffn_block(res, att, *tail)
+    for m in range(0, M, 16):
+        assert torch.equal(_lib.ffn_block(res[m:m + 16], att[m:m + 16], *tail), y[m:m + 16]), f"rows {m}.."
+
+
 @pytest.mark.parametrize("H", WIDTHS)
 def test_norms(H):
     dev = torch.device("cuda:0")
