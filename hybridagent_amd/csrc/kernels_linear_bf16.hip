@@ -37,16 +37,19 @@ hipError_t launch_linear_bf16(int epi, const uint16_t* x, const uint16_t* W, con
   const int64_t gy = lin_grid_y(M);
   if (gy > 65535) return hipErrorInvalidValue;
   const dim3 grid((unsigned)lin_grid_x(epi, N), (unsigned)gy), block(kLinThreads);
-#define W4A16_LIN(MT_)                                                                     \
-  do {                                                                                     \
-    switch (epi) {                                                                         \
-      case kLinGelu: hipLaunchKernelGGL((k_linear_bf16<MT_, kLinGelu>), grid, block, 0, s, a); break; \
-      case kLinResidual: hipLaunchKernelGGL((k_linear_bf16<MT_, kLinResidual>), grid, block, 0, s, a); break; \
-      case kLinGateUp: hipLaunchKernelGGL((k_linear_bf16<MT_, kLinGateUp>), grid, block, 0, s, a); break; \
-      case kLinGateUpFrag: hipLaunchKernelGGL((k_linear_bf16<MT_, kLinGateUpFrag>), grid, block, 0, s, a); break; \
-      case kLinPlainFrag: hipLaunchKernelGGL((k_linear_bf16<MT_, kLinPlainFrag>), grid, block, 0, s, a); break; \
-      default: hipLaunchKernelGGL((k_linear_bf16<MT_, kLinPlain>), grid, block, 0, s, a); break; \
-    }                                                                                      \
+  // the FFN block's fragment order comes from two row tiles on
+  if ((epi == kLinGateUpFrag || epi == kLinPlainFrag) && mt == 1) return hipErrorInvalidValue;
+#define W4A16_LIN1(MT_, EPI_) hipLaunchKernelGGL((k_linear_bf16<MT_, EPI_>), grid, block, 0, s, a)
+#define W4A16_LIN(MT_)                                     \
+  do {                                                     \
+    switch (epi) {                                         \
+      case kLinGelu: W4A16_LIN1(MT_, kLinGelu); break;     \
+      case kLinResidual: W4A16_LIN1(MT_, kLinResidual); break; \
+      case kLinGateUp: W4A16_LIN1(MT_, kLinGateUp); break; \
+      case kLinGateUpFrag: W4A16_LIN1(MT_ == 1 ? 2 : MT_, kLinGateUpFrag); break; \
+      case kLinPlainFrag: W4A16_LIN1(MT_ == 1 ? 2 : MT_, kLinPlainFrag); break; \
+      default: W4A16_LIN1(MT_, kLinPlain); break;          \
+    }                                                      \
   } while (0)
   if (mt == 1)
     W4A16_LIN(1);
@@ -55,6 +58,7 @@ hipError_t launch_linear_bf16(int epi, const uint16_t* x, const uint16_t* W, con
   else
     W4A16_LIN(4);
 #undef W4A16_LIN
+#undef W4A16_LIN1
   return hipGetLastError();
 }
 

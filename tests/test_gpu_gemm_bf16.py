@@ -68,6 +68,25 @@ def test_bf16_experts_segments(dev, H, I):
         assert ((got[t] - ref).abs() <= slack).all(), f"expert {e} of {ROWS[e]} rows"
 
 
+# at most 192 routed rows: the streaming kernel's chunks of 16, 32 and 64 rows
+@pytest.mark.parametrize("rows", [[3, 15, 16, 17, 0, 2, 33, 40], [1, 31, 32, 33, 40, 0], [63, 64, 65]])
+def test_bf16_experts_streamed_segments(dev, rows):
+    E, H, I = len(rows), 256, 160
+    g = torch.Generator(device=dev).manual_seed(31)
+    gu = (torch.randn(E, 2 * I, H, generator=g, device=dev) / math.sqrt(H)).to(torch.bfloat16)
+    dn = (torch.randn(E, H, I, generator=g, device=dev) / math.sqrt(I)).to(torch.bfloat16)
+    idx = torch.repeat_interleave(torch.arange(E), torch.tensor(rows))
+    idx = idx[torch.randperm(idx.numel(), generator=torch.Generator().manual_seed(32))]
+    M = idx.numel()
+    x = synth.activations(M, H, seed=33, device=dev)
+    got = _lib.bf16_experts_forward(x, idx[:, None].to(dev), torch.ones(M, 1, device=dev), gu, dn).double()
+    for e in range(E):
+        t = (idx == e).nonzero()[:, 0].to(dev)
+        if t.numel() > 0:
+            ref, slack = _mlp64(x[t].double(), gu[e, :I].double(), gu[e, I:].double(), dn[e].double())
+            assert ((got[t] - ref).abs() <= slack).all(), f"expert {e} of {rows[e]} rows"
+
+
 @pytest.mark.parametrize("H,I", [(256, 192), (160, 160)])
 def test_bf16_experts_two_slots_and_invalid(dev, H, I):
     # token-slot gathers (row / top_k) and slots without an expert, against the same routing on fp64
