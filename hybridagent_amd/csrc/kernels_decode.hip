@@ -146,8 +146,19 @@ constexpr int kSortWavesMax = 16;  // wavefronts of the wide form
 // chip idle while the others walk a whole expert; three each, in two rounds,
 // walk two thirds of one, a second stage included (193 tokens x top-8 at the
 // Gemma shape, G = 32, about 140 slots: the layer 149 -> 134 us tiled, 184 ->
-// 161 us packed; 128 tokens 146 -> 130 us).
+// 161 us packed; 128 tokens 146 -> 130 us).  Compiled in only where the
+// launcher may ask for it (two_rounds): its scalar work comes before a slot's
+// first load (a dense 2816 x 704 call of 4 rows 5.1 us with it, 4.8 without).
+template <int MODE, int KSPLIT, int SELF>
+constexpr bool two_rounds() {
+  return MODE == kModeGateUp && KSPLIT == 4 && SELF != kSelfRoute;
+}
+template <bool TWO>
 __host__ __device__ __forceinline__ int slot_wgs(const DecodeArgs& a, int U, int grid) {
+  if (!TWO) {
+    const int n = grid / U;
+    return n < 1 ? 1 : n < a.n_ct ? n : a.n_ct;
+  }
   if (a.resident > 0 && 2 * U > a.resident && 3 * U <= grid && 3 * U <= 2 * a.resident) return a.n_ct < 3 ? a.n_ct : 3;
   const int n = (a.resident > 0 && a.resident < grid ? (a.resident > U ? a.resident : U) : grid) / U;
   return n < 1 ? 1 : n < a.n_ct ? n : a.n_ct;
@@ -159,6 +170,7 @@ __global__ __launch_bounds__(stream_threads(KSPLIT)) __attribute__((amdgpu_waves
 void k_decode(DecodeArgs a) {
   constexpr int kStreamThreads = stream_threads(KSPLIT);  // the wide form
   constexpr int NWAVES = kStreamThreads / 64;
+  constexpr bool kTwo = two_rounds<MODE, KSPLIT, SELF>();
   const int CG = a.cg;  // column groups per item: 4 (wide) or 1 (narrow)
   extern __shared__ __align__(16) unsigned char smem_raw[];
   u32x4_t* __restrict__ lds_a = reinterpret_cast<u32x4_t*>(smem_raw);
@@ -373,7 +385,7 @@ void k_decode(DecodeArgs a) {
     // this workgroup's slot (the arithmetic below), its expert (the one whose
     // slots hold it), its 16-row chunk and the chunk's tokens, in the sort's
     // order; workgroups past the slots return below
-    const int wps_p = U == ug ? a.wps_guess : slot_wgs(a, U, (int)gridDim.x - 1);
+    const int wps_p = U == ug ? a.wps_guess : slot_wgs<kTwo>(a, U, (int)gridDim.x - 1);
     const int slot_p = U == ug ? slot_raw : (int)blockIdx.x / wps_p;
     if (slot_p < U) {
       if (tid < E && pslot[tid] <= slot_p && slot_p < pslot[tid + 1]) psel = tid;
@@ -395,7 +407,7 @@ void k_decode(DecodeArgs a) {
   }
   const bool guessed = U == ug;  // dense: always (u_guess is its slot count)
   const int work_grid = (int)gridDim.x - (SELF != kSelfNone ? 1 : 0);
-  const int wps = guessed ? a.wps_guess : slot_wgs(a, U, work_grid);
+  const int wps = guessed ? a.wps_guess : slot_wgs<kTwo>(a, U, work_grid);
   const int slot = guessed ? slot_raw : (int)blockIdx.x / wps;
   const int part = (int)blockIdx.x - slot * wps;
   if (slot >= U) return;  // uniform across the workgroup
@@ -905,7 +917,7 @@ static hipError_t launch_stream(DecodeArgs a, int ncolblk, int max_slots, hipStr
   // without them, 96 tokens of skewed routing (145 slots) 144 -> 126 us.
   constexpr int64_t kTwoRoundRows = SELF == kSelfPlan ? 896 : 768;
   a.resident = 0;
-  if (MODE == kModeGateUp && KSPLIT == 4 && SELF != kSelfRoute && !narrow && per_cu == 1 &&
+  if (two_rounds<MODE, KSPLIT, SELF>() && !narrow && per_cu == 1 &&
       2 * (int64_t)max_slots > resident && (int64_t)a.M * a.topk >= kTwoRoundRows) {
     a.resident = (int)resident;
     grid = std::max<int64_t>(grid, std::min<int64_t>(2 * resident, 3 * (int64_t)max_slots));
@@ -916,7 +928,7 @@ static hipError_t launch_stream(DecodeArgs a, int ncolblk, int max_slots, hipStr
   // differs; slot_magic = floor(2^32 / wps) + 1 gives blockIdx.x / wps
   // exactly for blockIdx.x < 2^16
   a.u_guess = std::max(max_slots, 1);
-  a.wps_guess = slot_wgs(a, a.u_guess, (int)grid);
+  a.wps_guess = slot_wgs<two_rounds<MODE, KSPLIT, SELF>()>(a, a.u_guess, (int)grid);
   a.slot_magic = a.wps_guess > 1 ? (uint32_t)((1ull << 32) / (uint64_t)a.wps_guess + 1ull) : 0u;
   a.per_guess = (a.n_ct + a.wps_guess - 1) / a.wps_guess;
   // SELF: one more workgroup, the last, writes the plan
