@@ -124,6 +124,7 @@ inline hipError_t launch_linear_call(const LinearCall& l, hipStream_t s) {
     a.M = (int)l.M;
     a.cols = l.N;
     a.K = l.K;
+    a.ranges = kLinRanges;
     a.mb = gemm_bf16_blocks(l.M, l.epi == kLinGateUp ? 2 * (int64_t)l.N : l.N);
     return launch_gemm_bf16(l.epi == kLinGateUp ? kGemmGateUp : kGemmPlain, a, 0, s);
   }
@@ -1080,6 +1081,7 @@ int moe_bf16_experts_forward(const uint16_t* hidden, const int64_t* topk_idx, co
     g.cols = (int)I;
     g.K = (int)H;
     g.queue = L.queues;
+    g.ranges = kBfGateUpRanges;
     const int mt = max_mtiles(M, top_k, E);
     if (e == hipSuccess) e = launch_gemm_bf16(kGemmGateUp, g, mt, s);
     g.act = L.inter;
@@ -1090,6 +1092,7 @@ int moe_bf16_experts_forward(const uint16_t* hidden, const int64_t* topk_idx, co
     g.cols = (int)H;
     g.K = (int)I;
     g.queue = L.queues + kPrefillQueueInts / 2;
+    g.ranges = kBfDownRanges;
     if (e == hipSuccess) e = launch_gemm_bf16(kGemmPlain, g, mt, s);
     if (e == hipSuccess) e = launch_combine(L.dn, topk_idx, topk_w, out, (int)M, (int)top_k, (int)E, (int)H, s);
     return launch_status(e);

@@ -37,6 +37,7 @@ constexpr int kBfMaxSteps = 12;  // 32-wide k steps per wavefront per chunk
 template <int MODE, int MT, int CB>
 __global__ __launch_bounds__(64 * kBfWaves) void k_bf16_expert(Bf16ExpertArgs a) {
   constexpr int KS = kBfWaves / CB;
+  static_assert(KS == (MODE == kModeGateUp ? kBfGateUpRanges : kBfDownRanges), "the ranges of a sum");
   __shared__ f32x4_t red[kBfWaves][MT][64];
   __shared__ int rowsrc[16 * MT];
   const int slot = blockIdx.y;

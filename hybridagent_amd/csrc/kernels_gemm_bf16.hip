@@ -24,10 +24,16 @@
 // the A operand (each lane ends with four consecutive output columns of one
 // row per register quad).  Step s of a stage takes k = 16 s .. 16 s + 15, so
 // a last half stage (K % 64 == 32) is two steps, and its loads of chunks
-// past K are turned to the row's chunk four before.  Each fragment register is reloaded for the next step right
-// after its last MFMA.  WM = 1: every wavefront has 32 weight rows x all MB
-// blocks of 32 activation rows; WM = 2: 64 weight rows x half of the rows,
-// which reads (MB + 2) fragments for 2 MB MFMAs instead of (MB + 1) for MB.
+// past K are turned to the row's chunk four before.  Each fragment register
+// is reloaded for the next step right after its last MFMA.  WM = 1: every
+// wavefront has 32 weight rows x all MB blocks of 32 activation rows; WM = 2:
+// 64 weight rows x half of the rows, which reads (MB + 2) fragments for 2 MB
+// MFMAs instead of (MB + 1) for MB.
+//
+// The dense kernels are built per tile height.  The accumulators of a range
+// and of the ranges before it are 160 registers at five blocks; they fit (no
+// spills) because one path leads through the last stage, whole or half: two
+// paths made the compiler hold a third set across their join.
 //
 // A workgroup goes from tile to tile without draining the ring: the next
 // tile's first two stages are issued before the current one's epilogue.
@@ -36,8 +42,15 @@
 // every XCD a contiguous run of tiles, ordered so that the tiles running at
 // once on an XCD share rows and columns.
 //
-// Every output is summed over k in order in one fp32 accumulator per element,
-// whatever tile it falls in.
+// Every output is the streaming kernels' sum, bit for bit, whatever tile it
+// falls in: K in the same ranges (GemmBf16Args::ranges), each range one fp32
+// chain, the ranges added in order -- so a row's result does not change where a
+// larger batch takes this kernel.  One 32x32x16 MFMA on chunks 0, 1 and one on
+// chunks 2, 3 of 32 k give the bits of the 16x16x32 MFMA on all four (compared
+// on 65,536 sums; every other order of the chunks differs).  A range's end
+// costs 32 VALU per block of 32 rows and group of 32 weight rows: against one
+// chain over all of K the FFN block at 2048 rows takes 492.8 us, not 490.4,
+// and 1031 tokens of BF16 experts 380.5, not 379.5.
 //
 // Bound: the experts by their weights' stream (1031 tokens x top-8, 128
 // experts of 11.9 MB: 1.64 ms streamed per 64 rows, 0.38 ms here, 4.1 TB/s
@@ -222,20 +235,28 @@ __device__ __forceinline__ int gx_run(const GemmBf16Args& a, unsigned char* smem
   constexpr int GC = GU ? 16 : 32;  // output columns of a 32-row weight group
   const bool work = ncol0 + GC * NB * wn < a.cols;
 
-  f32x16_t acc[NB][MB];
+  // acc: the current range of k, tot: the ranges before it
+  f32x16_t acc[NB][MB], tot[NB][MB];
 #pragma unroll
   for (int n = 0; n < NB; ++n)
 #pragma unroll
     for (int m = 0; m < MB; ++m)
 #pragma unroll
-      for (int q = 0; q < 16; ++q) acc[n][m][q] = 0.f;
+      for (int q = 0; q < 16; ++q) acc[n][m][q] = tot[n][m][q] = 0.f;
+  int left = a.krange;
+  auto add_range = [&] {
+#pragma unroll
+    for (int n = 0; n < NB; ++n)
+#pragma unroll
+      for (int m = 0; m < MB; ++m)
+#pragma unroll
+        for (int q = 0; q < 16; ++q) {
+          tot[n][m][q] += acc[n][m][q];
+          acc[n][m][q] = 0.f;
+        }
+    left = a.krange;
+  };
   u32x4_t af[MB], bf[NB], bn[NB];
-  auto read_a = [&](const unsigned char* st, int m, int s) {
-    return *reinterpret_cast<const u32x4_t*>(st + a0 + m * 4096 + off[s]);
-  };
-  auto read_b = [&](const unsigned char* st, int n, int s) {
-    return *reinterpret_cast<const u32x4_t*>(st + b0 + n * 4096 + off[s]);
-  };
   auto wait_and_sync = [&](int n, auto hook) {
     __builtin_amdgcn_sched_barrier(0);
     px_wait_vm(n);
@@ -251,92 +272,96 @@ __device__ __forceinline__ int gx_run(const GemmBf16Args& a, unsigned char* smem
   if (work) {
     const unsigned char* st = smem + slot * kGxStageBytes;
 #pragma unroll
-    for (int n = 0; n < NB; ++n) bf[n] = read_b(st, n, 0);
+    for (int n = 0; n < NB; ++n) bf[n] = *reinterpret_cast<const u32x4_t*>(st + b0 + n * 4096 + off[0]);
 #pragma unroll
-    for (int m = 0; m < MB; ++m) af[m] = read_a(st, m, 0);
+    for (int m = 0; m < MB; ++m) af[m] = *reinterpret_cast<const u32x4_t*>(st + a0 + m * 4096 + off[0]);
   }
-  // one stage of NS steps: refill the slot the stage before used
-  // (issue(slot2, part)), multiply, wait until at most n loads are in flight
-  // and meet the other wavefronts
-  auto stage = [&](auto ns, auto last, int n, auto issue, auto hook) {
-    constexpr int NS = decltype(ns)::value;
-    constexpr bool LAST = decltype(last)::value;
+  // one step: multiply the fragments at hand, reading the next step's (o: its
+  // place in the stage at st) behind the MFMAs that used them
+  auto step = [&](const unsigned char* st, int o) {
+#pragma unroll
+    for (int nn = 0; nn < NB; ++nn) bn[nn] = *reinterpret_cast<const u32x4_t*>(st + b0 + nn * 4096 + o);
+#pragma unroll
+    for (int m = 0; m < MB; ++m) {
+#pragma unroll
+      for (int nn = 0; nn < NB; ++nn) acc[nn][m] = mfma32(bf[nn], af[m], acc[nn][m]);
+      af[m] = *reinterpret_cast<const u32x4_t*>(st + a0 + m * 4096 + o);
+    }
+#pragma unroll
+    for (int nn = 0; nn < NB; ++nn) bf[nn] = bn[nn];
+  };
+  // one stage: refill the slot the stage before used (issue(slot2, part)),
+  // multiply, wait until at most n loads are in flight and meet the other
+  // wavefronts; the last step runs beside the next stage's first reads
+  auto stage = [&](int n, auto issue) {
     const int nslot = slot == kGxStages - 1 ? 0 : slot + 1;
     if (work) {
       const unsigned char* st = smem + slot * kGxStageBytes;
 #pragma unroll
-      for (int s = 0; s < NS - 1; ++s) {
+      for (int s = 0; s < 3; ++s) {
         issue(slot2, s);
-#pragma unroll
-        for (int nn = 0; nn < NB; ++nn) bn[nn] = read_b(st, nn, s + 1);
-#pragma unroll
-        for (int m = 0; m < MB; ++m) {
-#pragma unroll
-          for (int nn = 0; nn < NB; ++nn) acc[nn][m] = mfma32(bf[nn], af[m], acc[nn][m]);
-          af[m] = read_a(st, m, s + 1);
-        }
-#pragma unroll
-        for (int nn = 0; nn < NB; ++nn) bf[nn] = bn[nn];
+        step(st, off[s + 1]);
+        if (s == 1 && --left == 0) add_range();
       }
-#pragma unroll
-      for (int p = NS - 1; p < 4; ++p) issue(slot2, p);
-      wait_and_sync(n, hook);
-      const unsigned char* sn = smem + nslot * kGxStageBytes;
-      if (!LAST) {
-#pragma unroll
-        for (int nn = 0; nn < NB; ++nn) bn[nn] = read_b(sn, nn, 0);
-      }
-#pragma unroll
-      for (int m = 0; m < MB; ++m) {
-#pragma unroll
-        for (int nn = 0; nn < NB; ++nn) acc[nn][m] = mfma32(bf[nn], af[m], acc[nn][m]);
-        if (!LAST) af[m] = read_a(sn, m, 0);
-      }
-      if (!LAST) {
-#pragma unroll
-        for (int nn = 0; nn < NB; ++nn) bf[nn] = bn[nn];
-      }
+      issue(slot2, 3);
+      wait_and_sync(n, no_hook);
+      step(smem + nslot * kGxStageBytes, off[0]);
+      if (--left == 0) add_range();
     } else {
 #pragma unroll
       for (int p = 0; p < 4; ++p) issue(slot2, p);
-      wait_and_sync(n, hook);
+      wait_and_sync(n, no_hook);
     }
     slot = nslot;
     slot2 = slot2 == kGxStages - 1 ? 0 : slot2 + 1;
   };
-  std::integral_constant<int, 4> full;
-  std::integral_constant<int, 2> half;
   {
     const GxLoads lc = gx_loads<EPI, GROUPED>(a, it, smem);
     for (int t = 0; t + 2 < nkt; ++t)
-      stage(full, std::false_type{}, lc.na + kGxNB,
-            [&](int sl, int p) { gx_issue<EPI>(a, lc, smem, t + 2, sl, p); }, no_hook);
+      stage(lc.na + kGxNB, [&](int sl, int p) { gx_issue<EPI>(a, lc, smem, t + 2, sl, p); });
   }
   // no stage loads are left for the last two stages: the first of them brings
   // the row indices (gate/up: the next tile's rows, for its load sources;
   // plain: this tile's output rows)
   const bool tab = GROUPED && wave == 0;  // wavefront-uniform
-  stage(full, std::false_type{}, tab ? 1 : 0, [&](int, int p) {
+  stage(tab ? 1 : 0, [&](int, int p) {
     if (p == 0 && tab) {
       const int tseg = GU && has_next ? nx.seg0 : it.seg0;
       px_dma16(make_rsrc(a.sorted_pos, (uint32_t)a.rows_total * 4u), 4 * ((tseg & ~3) + 4 * lane), 0, smem + kGxTable);
     }
-  }, no_hook);
+  });
+  // the last stage, whole or half: where it is whole its first two steps, then
+  // the two steps both have (one path for the accumulators)
+  const bool whole = a.K % kGxKT == 0;
   const bool fetch = GROUPED && fetch_q != nullptr && wave == 0;  // wavefront-uniform
   int fv = 0;
-  auto take = [&](int, int p) {
-    if (p == 0 && fetch && lane == 0)
-      fv = __hip_atomic_fetch_add(fetch_q, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  };
-  auto put = [&] {
+  if (fetch && lane == 0) fv = __hip_atomic_fetch_add(fetch_q, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (work) {
+    const unsigned char* st = smem + slot * kGxStageBytes;
+    if (whole) {
+      step(st, off[1]);
+      step(st, off[2]);
+      if (--left == 0) add_range();
+    }
+    step(st, whole ? off[3] : off[1]);
+  }
+  wait_and_sync(0, [&] {
     if (fetch && lane == 0) *reinterpret_cast<int*>(smem + kGxQSlot) = fv;
-  };
-  if (a.K % kGxKT != 0)
-    stage(half, std::true_type{}, 0, take, put);
-  else
-    stage(full, std::true_type{}, 0, take, put);
+  });
+  if (work) {
+#pragma unroll
+    for (int m = 0; m < MB; ++m)
+#pragma unroll
+      for (int nn = 0; nn < NB; ++nn) acc[nn][m] = mfma32(bf[nn], af[m], acc[nn][m]);
+  }
   const int n_next = has_next ? gx_issue_first<EPI, GROUPED>(a, nx, smem, (p0 + nkt) % kGxStages) : 0;
   if (!work) return n_next;
+#pragma unroll
+  for (int n = 0; n < NB; ++n)
+#pragma unroll
+    for (int m = 0; m < MB; ++m)
+#pragma unroll
+      for (int q = 0; q < 16; ++q) tot[n][m][q] += acc[n][m][q];
 
   // ---- epilogue: lane (h, c) holds, for row 32 m + c of its block, weight
   // rows 8 J + 4 h + i of group n in acc[n][m][4 J + i]
@@ -356,8 +381,8 @@ __device__ __forceinline__ int gx_run(const GemmBf16Args& a, unsigned char* smem
           float hv[4];
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            const float g = round_bf16(acc[n][m][4 * J + i]);
-            const float u = round_bf16(acc[n][m][4 * J + i + 8]);
+            const float g = round_bf16(tot[n][m][4 * J + i]);
+            const float u = round_bf16(tot[n][m][4 * J + i + 8]);
             hv[i] = round_bf16(gelu_tanh_f32(g)) * u;
           }
           *reinterpret_cast<uint2*>(orow + 8 * J) = make_uint2(pack_bf16x2(hv[0], hv[1]), pack_bf16x2(hv[2], hv[3]));
@@ -377,8 +402,8 @@ __device__ __forceinline__ int gx_run(const GemmBf16Args& a, unsigned char* smem
 #pragma unroll
         for (int J = 0; J < 4; ++J)
           *reinterpret_cast<uint2*>(ob + c * kGxEpiPitch + 2 * (8 * J + 4 * h)) =
-              make_uint2(pack_bf16x2(acc[n][m][4 * J], acc[n][m][4 * J + 1]),
-                         pack_bf16x2(acc[n][m][4 * J + 2], acc[n][m][4 * J + 3]));
+              make_uint2(pack_bf16x2(tot[n][m][4 * J], tot[n][m][4 * J + 1]),
+                         pack_bf16x2(tot[n][m][4 * J + 2], tot[n][m][4 * J + 3]));
         const int col = ncol0 + 32 * (wn * NB + n);
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
@@ -396,17 +421,21 @@ __device__ __forceinline__ int gx_run(const GemmBf16Args& a, unsigned char* smem
   return n_next;
 }
 
-template <int EPI, bool GROUPED>
+// MBD: dense, the launch's row blocks per tile (0: grouped)
+template <int EPI, int MBD>
 __device__ __forceinline__ int gx_dispatch(const GemmBf16Args& a, unsigned char* smem, const GxItem& it,
                                            const GxItem& nx, bool has_next, int p0, int n_inflight, int* fetch_q) {
+  constexpr bool GROUPED = MBD == 0;
+  if constexpr (!GROUPED) {
+    // wavefronts by rows where that reads fewer fragments per MFMA
+    constexpr int WM = MBD == 2 || MBD == 4 ? 2 : 1;
+    return gx_run<EPI, GROUPED, MBD / WM, WM>(a, smem, it, nx, has_next, p0, n_inflight, fetch_q);
+  }
   switch (it.mb) {
     case 1: return gx_run<EPI, GROUPED, 1, 1>(a, smem, it, nx, has_next, p0, n_inflight, fetch_q);
     case 2: return gx_run<EPI, GROUPED, 1, 2>(a, smem, it, nx, has_next, p0, n_inflight, fetch_q);
     case 3: return gx_run<EPI, GROUPED, 3, 1>(a, smem, it, nx, has_next, p0, n_inflight, fetch_q);
-    case 4: return gx_run<EPI, GROUPED, 2, 2>(a, smem, it, nx, has_next, p0, n_inflight, fetch_q);
-    default:
-      if constexpr (!GROUPED) return gx_run<EPI, GROUPED, 5, 1>(a, smem, it, nx, has_next, p0, n_inflight, fetch_q);
-      return 0;
+    default: return gx_run<EPI, GROUPED, 2, 2>(a, smem, it, nx, has_next, p0, n_inflight, fetch_q);
   }
 }
 
@@ -416,9 +445,10 @@ __device__ __forceinline__ int gx_dispatch(const GemmBf16Args& a, unsigned char*
 // have left; the sort zeroes the counters and the last to leave resets them.
 // Dense: XCD x has tiles [x per, x per + per) in order, its workgroups every
 // P-th of them.
-template <int EPI, bool GROUPED>
+template <int EPI, int MBD>
 __global__ __launch_bounds__(kGxThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void k_gemm_bf16(GemmBf16Args a) {
+  constexpr bool GROUPED = MBD == 0;
   extern __shared__ __align__(16) unsigned char smem[];
   int item, end, step;
   if (GROUPED) {
@@ -460,7 +490,7 @@ void k_gemm_bf16(GemmBf16Args a) {
   for (;;) {
     const bool has_next = nitem < end;
     const GxItem nxt = has_next ? gx_item<GROUPED>(a, nitem) : cur;
-    n_inflight = gx_dispatch<EPI, GROUPED>(a, smem, cur, nxt, has_next, p0, n_inflight, has_next ? a.queue : nullptr);
+    n_inflight = gx_dispatch<EPI, MBD>(a, smem, cur, nxt, has_next, p0, n_inflight, has_next ? a.queue : nullptr);
     if (!has_next) break;
     nitem = GROUPED ? 2 * step + __builtin_amdgcn_readfirstlane(*reinterpret_cast<volatile int*>(smem + kGxQSlot))
                     : nitem + step;
@@ -507,21 +537,26 @@ hipError_t launch_gemm_bf16(int epi, GemmBf16Args a, int max_items, hipStream_t 
     items = (((int64_t)a.M + 32 * a.mb - 1) / (32 * a.mb)) * a.n_nt;
   }
   if (items <= 0) return hipSuccess;
+  if (a.ranges < 1) return hipErrorInvalidValue;
+  a.krange = (a.K / 32 + a.ranges - 1) / a.ranges;
   if (items > (int64_t(1) << 30)) return hipErrorInvalidValue;
-#define W4A16_GX(EPI_, G_)                                                                                       \
-  do {                                                                                                           \
-    auto kern = k_gemm_bf16<EPI_, G_>;                                                                           \
-    hipLaunchKernelGGL(kern, dim3(prefill_grid_size(reinterpret_cast<const void*>(kern), kGxThreads, kGxLds,     \
-                                                    (int)items)),                                                \
-                       dim3(kGxThreads), kGxLds, s, a);                                                          \
-  } while (0)
-  if (epi == kGemmGateUp) {
-    if (grouped) W4A16_GX(kGemmGateUp, true);
-    else W4A16_GX(kGemmGateUp, false);
-  } else {
-    if (grouped) W4A16_GX(kGemmPlain, true);
-    else W4A16_GX(kGemmPlain, false);
+  auto launch = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3(prefill_grid_size(reinterpret_cast<const void*>(kern), kGxThreads, kGxLds, (int)items)),
+                       dim3(kGxThreads), kGxLds, s, a);
+  };
+#define W4A16_GX(EPI_)                              \
+  switch (grouped ? 0 : a.mb) {                     \
+    case 0: launch(k_gemm_bf16<EPI_, 0>); break;    \
+    case 1: launch(k_gemm_bf16<EPI_, 1>); break;    \
+    case 2: launch(k_gemm_bf16<EPI_, 2>); break;    \
+    case 3: launch(k_gemm_bf16<EPI_, 3>); break;    \
+    case 4: launch(k_gemm_bf16<EPI_, 4>); break;    \
+    default: launch(k_gemm_bf16<EPI_, 5>); break;   \
   }
+  if (epi == kGemmGateUp)
+    W4A16_GX(kGemmGateUp)
+  else
+    W4A16_GX(kGemmPlain)
 #undef W4A16_GX
   return hipGetLastError();
 }

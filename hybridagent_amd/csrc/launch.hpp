@@ -303,6 +303,12 @@ hipError_t launch_bf16_experts(int mode, Bf16ExpertArgs a, int max_slots, hipStr
 bool linear_w4_supported(int64_t M, int64_t N, int64_t K, int64_t G);
 hipError_t launch_linear_w4(const uint16_t* x, const int32_t* wp, const uint16_t* ws, const uint16_t* bias,
                             uint16_t* y, int64_t M, int64_t N, int64_t K, int64_t G, hipStream_t s);
+// K ranges of the streaming bf16 kernels' sums (k_linear_bf16; k_bf16_expert's
+// two projections): a sum is the ranges' fp32 chains, each ceil(K / 32 /
+// ranges) steps of 32, added in order.  The prefill GEMM forms the same sums.
+constexpr int kLinRanges = 8;
+constexpr int kBfGateUpRanges = 4;
+constexpr int kBfDownRanges = 2;
 // bf16 x bf16 GEMMs at prefill sizes (kernels_gemm_bf16.hip)
 enum GemmEpilogue { kGemmGateUp = 0, kGemmPlain = 1 };
 struct GemmBf16Args {
@@ -314,12 +320,13 @@ struct GemmBf16Args {
   int cols, K;
   int64_t wrows;              // grouped: weight rows per expert
   int mb;                     // dense: 32-row blocks per tile, 1 .. 5
+  int ranges;                 // K ranges of a sum (the streaming kernel's)
   // grouped (tiles non-null): the plan's 128-row tiles, its segment starts,
   // positions and counters, the queue (9 ints, zero) and the routed rows
   const int32_t *sorted_pos, *offsets, *tiles, *counters;
   int32_t* queue;
   int topk, rows_total;
-  int n_nt;                   // set by the launcher: column tiles
+  int n_nt, krange;           // set by the launcher: column tiles, 32-wide steps per range
 };
 // K a multiple of 32 above 128, cols a multiple of 32
 bool gemm_bf16_supported(int64_t K, int64_t cols);

@@ -20,7 +20,7 @@
 
 namespace w4a16 {
 
-constexpr int kLinWaves = 8;
+constexpr int kLinWaves = kLinRanges;  // a range of K each
 constexpr int kLinThreads = 64 * kLinWaves;
 constexpr int kLinMaxSteps = 12;  // 32-wide k steps per wavefront held in registers
 
