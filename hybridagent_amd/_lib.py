@@ -195,7 +195,7 @@ def _bf16(t: torch.Tensor, name: str) -> torch.Tensor:
 
 def _rows(t: torch.Tensor, width: int) -> torch.Tensor:
     """t as a matrix of rows of `width` (t itself if it is one)."""
-    return t if t.dim() == 2 else t.reshape(-1, width)
+    return t if t.dim() == 2 and t.shape[1] == width else t.reshape(-1, width)
 
 
 def _like(out: torch.Tensor, shape) -> torch.Tensor:
