@@ -4,6 +4,7 @@
 #include "w4a16moe.h"
 
 #include "launch.hpp"
+#include "rules.hpp"
 #include <algorithm>
 #include <atomic>
 #include <mutex>
@@ -80,18 +81,6 @@ struct AddNorm {
   uint16_t* y;
 };
 
-// Whether a shared-MLP linear (M rows, N output columns, K deep) runs as the
-// tiled GEMM instead of streaming its weights once per 64 rows
-// (k_linear_bf16).  A launch of few tiles takes a tile's time, about 20 us at
-// K = 2816, whatever its size; the stream's time grows with the weights and
-// the 64-row passes.  The FFN block (H = 2816), streamed / tiled, in us: Im =
-// 1056 at 96 / 128 / 160 rows 170/182, 218/219, 228/223; Im = 1600 at 81 / 96
-// 178/179, 185/183; Im = 2112 at 65 / 81 / 300 / 2048 181/187, 187/186,
-// 331/246, 1237/506; Im = 4096 at 65 211/204.
-inline bool linear_tiled(int64_t M, int64_t N, int64_t K) {
-  return M > 64 && M * N * K > 420000000 && gemm_bf16_supported(K, N);
-}
-
 // Whether Linear4Bit (M rows, N columns) runs as the tiled GEMM instead of
 // streaming its weights once per 16 rows (k_decode<dense>).  Few tiles take a
 // tile's time, which grows with K as the stream's does.  K = 2816, streamed /
@@ -115,7 +104,8 @@ struct FfnPost {
 };
 
 inline hipError_t launch_linear_call(const LinearCall& l, hipStream_t s) {
-  if ((l.epi == kLinGateUp || l.epi == kLinPlain) && linear_tiled(l.M, l.N, l.K)) {
+  if ((l.epi == kLinGateUp || l.epi == kLinPlain) && linear_tiled_rows(l.M, l.N, l.K) &&
+      gemm_bf16_supported(l.K, l.N)) {
     GemmBf16Args a{};
     a.act = l.x;
     a.W = l.W;
@@ -968,8 +958,8 @@ static int ffn_block_impl(const uint16_t* residual, const uint16_t* attn_out,
   // (top_k = 1, an Im above the experts' rows) the order stays row-major, so
   // the workspace is what it was.
   const int64_t mp = (M + 15) / 16 * 16;
-  const bool frag =
-      M > 16 && !linear_tiled(M, Im, H) && !linear_tiled(M, H, Im) && mp * (H + Im) <= M * top_k * H;
+  const bool frag = ffn_fragment_rows(M, H, Im, mp * (H + Im) <= M * top_k * H,
+                                      gemm_bf16_supported(H, Im) && gemm_bf16_supported(Im, H));
   uint16_t* const dn = moe_layout(L.moe_ws, M, top_k, E, H, I).dn;
   uint16_t* const h_ff = frag ? dn : L.h_ff;
   uint16_t* const inter = frag ? dn + mp * H : L.inter;

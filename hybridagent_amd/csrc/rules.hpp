@@ -1,0 +1,38 @@
+// Which kernel a call's bf16 linears run: host rules on sizes alone, free of
+// HIP so that they can be checked without a GPU.
+#pragma once
+#include <stdint.h>
+
+namespace w4a16 {
+
+// A shared-MLP linear (M rows, N output columns, K deep) as the tiled GEMM
+// instead of the stream (k_linear_bf16, its weights once per 64 rows).  A
+// launch of few tiles takes a tile's time, about 20 us at K = 2816, whatever
+// its size; the stream's grows with the 64-row passes and the weights of each.
+
+// The stream on rows in fragment order.  Two passes were never slower; from
+// the third on the line is passes times weights.  The FFN block (H = 2816),
+// streamed / tiled, in us, at 128, 129, 193..208, 257..288 rows: Im = 512
+// 158/173, 164/175, 194/202, 265/259; 1056 163/181, 169/182, 207/209, 240/236;
+// 1600 167/183, 201/207, 218/212, 253/238; 2112 176/189, 214/214, 229/217,
+// 273/244; 4096 199/208, 225/210, 276/235, 331/266; 12288 300/299, 360/322.
+inline bool linear_tiled_frag(int64_t M, int64_t N, int64_t K) {
+  return M > 128 && ((M + 63) / 64 - 2) * (N * K) > 4600000;
+}
+
+// The stream on row-major rows (16 x 64 bytes a load): tiled earlier.  Im =
+// 1056 at 96 / 128 / 160 rows 170/182, 218/219, 228/223; 1600 at 81 / 96
+// 178/179, 185/183; 2112 at 65 / 81 / 300 181/187, 187/186, 331/246; 4096 at
+// 65 211/204.
+inline bool linear_tiled_rows(int64_t M, int64_t N, int64_t K) {
+  return (M > 64 && M * N * K > 420000000) || linear_tiled_frag(M, N, K);
+}
+
+// The block's two linears (H x Im) stream fragment-order rows: from 17 rows
+// on, one row tile gains nothing; `fits`: the padded rows fit in the place
+// they are held.
+inline bool ffn_fragment_rows(int64_t M, int64_t H, int64_t Im, bool fits, bool tiles_supported) {
+  return M > 16 && fits && !(tiles_supported && linear_tiled_frag(M, Im, H));
+}
+
+}  // namespace w4a16

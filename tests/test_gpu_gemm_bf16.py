@@ -113,8 +113,8 @@ def test_bf16_experts_two_slots_and_invalid(dev, H, I):
     assert ((got - ref).abs() <= slack + 2.0 ** -8 * ref.abs()).all()
 
 
-# at H = 2816 the tiled GEMM takes more than 420e6 multiply-adds (M H Im): both sides of that, tiles' edges, half k
-# stages (Im % 64 == 32) and rows enough for every tile height of the dense launch
+# at H = 2816 the streams run up to 128 rows and, at Im = 1120 and 800, at 129 and 193; the others run tiles: their
+# edges, half k stages (Im % 64 == 32) and rows enough for every tile height of the dense launch
 @pytest.mark.parametrize("M,Im", [(65, 160), (81, 1056), (129, 1120), (193, 800), (257, 608), (300, 1056), (481, 2112),
                                   (700, 2112), (1025, 2112), (1700, 2112), (2047, 2112)])
 def test_ffn_shared_mlp_rows(dev, M, Im):
