@@ -21,7 +21,7 @@
 //
 // Bound: the dequantisation's VALU beside the MFMAs, and the last round of
 // tiles.  2816 x 2816, G = 32, at 512 / 1024 / 2048 / 4096 rows:
-// streamed 33 / 54 / 99 / 186 us, here 24 / 28 / 40 / 66 us (815 TFLOP/s at 2048).
+// streamed 33 / 54 / 99 / 186 us, here 24 / 28 / 40 / 64 us (815 TFLOP/s at 2048).
 #include <type_traits>
 
 #include "common.hpp"
@@ -146,8 +146,9 @@ void k_linear_w4(LinearW4Args a) {
     bw = *reinterpret_cast<const u32x4_t*>(st + boff);
     es = exact_scale(bf16_bits_to_f32(*reinterpret_cast<const uint16_t*>(srow + 2 * g)));
   };
-  // zero in the lanes of h = 1 (a last half stage has no k for them)
-  auto keep = [&](u32x4_t v) { return h ? u32x4_t{0u, 0u, 0u, 0u} : v; };
+  // zero in the lanes of h = 1 of a last half stage, which has no k for them
+  const bool none = odd && h != 0;
+  auto keep = [&](u32x4_t v) { return none ? u32x4_t{0u, 0u, 0u, 0u} : v; };
 
   px_wait_vm(na + 1);
   px_barrier();  // the scales and stage 0 landed (stage 1 may still be loading)
@@ -160,18 +161,21 @@ void k_linear_w4(LinearW4Args a) {
   // step right after its MFMA, the next step's word is dequantised beside the
   // current step's MFMAs, and the last step's MFMAs run after the barrier,
   // beside the next stage's first reads
-  auto stage = [&](int t, auto halfs, bool fill, int left) {
-    constexpr bool HALF = decltype(halfs)::value;  // a last half stage
+  // (LAST: the last stage, whole or half by a lane mask.  Two paths here made
+  // the compiler hold a second set of accumulators, 16 registers spilled at
+  // six blocks: 4096 rows of 704 x 2816 25.0 us against 22.1.)
+  auto stage = [&](int t, auto last, bool fill, int left) {
+    constexpr bool LAST = decltype(last)::value;
     const unsigned char* st = smem + slot * kStage;
     const int nslot = slot == kLwStages - 1 ? 0 : slot + 1;
 #pragma unroll
     for (int s = 0; s < 3; ++s) {
       if (fill) issue(t + 2, slot2, s);
       const u32x4_t bn = unpack_exact<false>(s == 0 ? bw.y : s == 1 ? bw.z : bw.w, es, kr);
-      const u32x4_t b = HALF ? keep(bf) : bf;
+      const u32x4_t b = LAST ? keep(bf) : bf;
 #pragma unroll
       for (int m = 0; m < MB; ++m) {
-        acc[m] = mfma32(b, HALF ? keep(af[m]) : af[m], acc[m]);
+        acc[m] = mfma32(b, LAST ? keep(af[m]) : af[m], acc[m]);
         af[m] = read_a(st, s + 1, m);
       }
       bf = bn;
@@ -180,8 +184,8 @@ void k_linear_w4(LinearW4Args a) {
     __builtin_amdgcn_sched_barrier(0);
     px_wait_vm(left);
     px_barrier();  // stage t + 1 landed
-    const u32x4_t b = HALF ? keep(bf) : bf;
-    if (t + 1 < nkt) {
+    const u32x4_t b = LAST ? keep(bf) : bf;
+    if (!LAST) {
       const unsigned char* sn = smem + nslot * kStage;
       read_b(sn, t + 1);
 #pragma unroll
@@ -192,17 +196,14 @@ void k_linear_w4(LinearW4Args a) {
       bf = unpack_exact<false>(bw.x, es, kr);
     } else {
 #pragma unroll
-      for (int m = 0; m < MB; ++m) acc[m] = mfma32(b, HALF ? keep(af[m]) : af[m], acc[m]);
+      for (int m = 0; m < MB; ++m) acc[m] = mfma32(b, LAST ? keep(af[m]) : af[m], acc[m]);
     }
     slot = nslot;
     slot2 = slot2 == kLwStages - 1 ? 0 : slot2 + 1;
   };
   for (int t = 0; t + 2 < nkt; ++t) stage(t, std::false_type{}, true, na + 1);
   stage(nkt - 2, std::false_type{}, false, 0);
-  if (odd)
-    stage(nkt - 1, std::true_type{}, false, 0);
-  else
-    stage(nkt - 1, std::false_type{}, false, 0);
+  stage(nkt - 1, std::true_type{}, false, 0);
 
   // Lane (h, c) holds, for row 32 m + c, weight rows 8 J + 4 h + i in
   // acc[m][4 J + i].  Every wavefront is past its last read of the ring, which

@@ -54,7 +54,7 @@ def kernels():
     return found
 
 
-@pytest.mark.parametrize("name", ["k_prefill_x", "k_gemm_bf16"])
+@pytest.mark.parametrize("name", ["k_prefill_x", "k_gemm_bf16", "k_linear_w4"])
 def test_no_vector_register_spills(kernels, name):
     mine = {n: k for n, k in kernels.items() if name in n}
     assert mine
