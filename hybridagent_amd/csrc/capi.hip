@@ -115,7 +115,7 @@ inline hipError_t launch_linear_call(const LinearCall& l, hipStream_t s) {
     a.cols = l.N;
     a.K = l.K;
     a.ranges = kLinRanges;
-    a.mb = gemm_bf16_blocks(l.M, l.epi == kLinGateUp ? 2 * (int64_t)l.N : l.N);
+    a.mb = gemm_bf16_blocks(l.M, l.epi == kLinGateUp ? 2 * (int64_t)l.N : l.N, device_cus());
     return launch_gemm_bf16(l.epi == kLinGateUp ? kGemmGateUp : kGemmPlain, a, 0, s);
   }
   return launch_linear_bf16(l.epi, l.x, l.W, l.W2, l.bias, l.res, l.out, l.M, l.N, l.K, s);
@@ -329,7 +329,7 @@ int w4a16_linear(const uint16_t* x, const int32_t* w_packed, const uint16_t* w_s
   (void)workspace_bytes;
   if (K > kMaxStreamK) return W4A16_ERR_SHAPE;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (linear_w4_tiled(M, N) && linear_w4_supported(M, N, K, group_size))
+  if (linear_w4_tiled(M, N) && linear_w4_supported(K, group_size))
     return launch_status(launch_linear_w4(x, w_packed, w_scale, bias, y, M, N, K, group_size, s));
   DecodeArgs a{};
   a.act = x;

@@ -61,6 +61,7 @@
 #include "common.hpp"
 #include "launch.hpp"
 #include "lds_pipe.hpp"
+#include "rules.hpp"
 
 namespace w4a16 {
 
@@ -68,9 +69,9 @@ namespace {
 
 constexpr int kGxWaves = 8;
 constexpr int kGxThreads = 64 * kGxWaves;
-constexpr int kGxBN = 256;      // weight rows per tile
-constexpr int kGxKT = 64;       // k per stage
-constexpr int kGxMaxBlocks = 5; // 32-row blocks per tile
+constexpr int kGxBN = 256;  // weight rows per tile
+constexpr int kGxKT = 64;   // k per stage
+constexpr int kGxMaxBlocks = kGemmMaxBlocks;  // 32-row blocks per tile
 constexpr int kGxStages = 3;
 // a stage: A [160 rows][128 B] | B [256 rows][128 B]; after the ring the row
 // indices of a grouped tile (256 ints from a 16-byte-aligned start) and the
@@ -504,27 +505,6 @@ bool gemm_bf16_supported(int64_t K, int64_t cols) {
   // three stages at least; whole 32-row weight groups (the gate/up form's 16
   // columns of a group among them) and 16-byte rows
   return K % 32 == 0 && K > 2 * kGxKT && cols % 32 == 0 && cols > 0 && K <= (1 << 20);
-}
-
-// The tile height of a dense launch.  All tiles of a launch are alike and one
-// workgroup runs per CU, so the time is the rounds of tiles (one per CU each)
-// times a tile's, which is close to (blocks + 1): its MFMAs, and a stage's
-// weights, barrier and waits whatever the height.  The FFN block at 2048 rows
-// with 1 .. 5 blocks: 610 / 566 / 522 / 530 / 511 us, with the height this
-// picks for each of its two linears 506 us.
-int gemm_bf16_blocks(int64_t M, int64_t wrows) {
-  const int64_t n_nt = (wrows + kGxBN - 1) / kGxBN;
-  int best = 1;
-  int64_t cost = 0;
-  for (int mb = 1; mb <= kGxMaxBlocks; ++mb) {
-    const int64_t tiles = (M + 32 * mb - 1) / (32 * mb) * n_nt;
-    const int64_t c = (tiles + 255) / 256 * (mb + 1);
-    if (mb == 1 || c < cost) {
-      best = mb;
-      cost = c;
-    }
-  }
-  return best;
 }
 
 hipError_t launch_gemm_bf16(int epi, GemmBf16Args a, int max_items, hipStream_t s) {

@@ -27,6 +27,7 @@
 #include "common.hpp"
 #include "launch.hpp"
 #include "lds_pipe.hpp"
+#include "rules.hpp"
 
 namespace w4a16 {
 
@@ -243,40 +244,26 @@ void k_linear_w4(LinearW4Args a) {
   }
 }
 
-// 32-row blocks per tile: the cheapest of the heights whose ring and scales
-// fit in LDS (0: none).  One workgroup runs per CU, so the time is the rounds
-// of tiles times a tile's; a tile of 1 .. 6 blocks measured 24, 27, 33, 34,
-// 41, 48 us at K = 2816 (a stage's barrier and waits dominate few blocks).
-static int linear_w4_blocks(int64_t M, int64_t N, int64_t ng) {
-  constexpr int kTileCost[6] = {24, 27, 33, 34, 41, 48};
-  const int64_t n_nt = (N + kLwBN - 1) / kLwBN;
-  int best = 0;
-  int64_t cost = 0;
-  for (int mb = 1; mb <= 6; ++mb) {
-    if (kLwStages * lw_stage(mb) + lw_scale_bytes((int)ng) > 160 * 1024) break;
-    const int64_t tiles = (M + 32 * mb - 1) / (32 * mb) * n_nt;
-    const int64_t c = (tiles + 255) / 256 * kTileCost[mb - 1];
-    if (best == 0 || c < cost) {
-      best = mb;
-      cost = c;
-    }
-  }
-  return best;
+// most 32-row blocks per tile whose ring and scales fit in LDS (0: none)
+static int linear_w4_max_blocks(int64_t ng) {
+  int mb = kLinearW4MaxBlocks;
+  while (mb > 0 && kLwStages * lw_stage(mb) + lw_scale_bytes((int)ng) > 160 * 1024) --mb;
+  return mb;
 }
 
-bool linear_w4_supported(int64_t M, int64_t N, int64_t K, int64_t G) {
+bool linear_w4_supported(int64_t K, int64_t G) {
   const int64_t ng = (K + G - 1) / G;
   // at least three stages
-  return K % 32 == 0 && K > 2 * kLwKT && K <= (1 << 20) && ng <= 1024 && linear_w4_blocks(M, N, ng) != 0;
+  return K % 32 == 0 && K > 2 * kLwKT && K <= (1 << 20) && ng <= 1024 && linear_w4_max_blocks(ng) > 0;
 }
 
 hipError_t launch_linear_w4(const uint16_t* x, const int32_t* wp, const uint16_t* ws, const uint16_t* bias,
                             uint16_t* y, int64_t M, int64_t N, int64_t K, int64_t G, hipStream_t s) {
   if (M == 0) return hipSuccess;
-  if (!linear_w4_supported(M, N, K, G)) return hipErrorInvalidValue;
+  if (!linear_w4_supported(K, G)) return hipErrorInvalidValue;
   LinearW4Args a{x, wp, ws, bias, y, (int)M, (int)N, (int)K, (int)((K + G - 1) / G), 0, 0, 0, 0};
   while ((int64_t(1) << (a.gshift + 1)) <= G) ++a.gshift;
-  const int mb = linear_w4_blocks(M, N, a.ng);
+  const int mb = linear_w4_blocks(M, N, device_cus(), linear_w4_max_blocks(a.ng));
   a.n_mt = (int)((M + 32 * mb - 1) / (32 * mb));
   a.n_nt = (int)((N + kLwBN - 1) / kLwBN);
   a.vec = N % 8 == 0 && (reinterpret_cast<uintptr_t>(y) & 15u) == 0;

@@ -300,7 +300,7 @@ hipError_t launch_ffn_post(const FfnPostCall& c, const uint16_t* moe, const int6
 hipError_t launch_bf16_experts(int mode, Bf16ExpertArgs a, int max_slots, hipStream_t s);
 // Linear4Bit at prefill sizes (kernels_linear_w4.hip): K a multiple of 32
 // above 128 whose scales fit in LDS
-bool linear_w4_supported(int64_t M, int64_t N, int64_t K, int64_t G);
+bool linear_w4_supported(int64_t K, int64_t G);
 hipError_t launch_linear_w4(const uint16_t* x, const int32_t* wp, const uint16_t* ws, const uint16_t* bias,
                             uint16_t* y, int64_t M, int64_t N, int64_t K, int64_t G, hipStream_t s);
 // K ranges of the streaming bf16 kernels' sums (k_linear_bf16; k_bf16_expert's
@@ -330,8 +330,6 @@ struct GemmBf16Args {
 };
 // K a multiple of 32 above 128, cols a multiple of 32
 bool gemm_bf16_supported(int64_t K, int64_t cols);
-// 32-row blocks per tile of a dense launch for M rows and `wrows` weight rows
-int gemm_bf16_blocks(int64_t M, int64_t wrows);
 // max_items: grouped, most m-tiles
 hipError_t launch_gemm_bf16(int epi, GemmBf16Args a, int max_items, hipStream_t s);
 // prefill grouped GEMM: one launch per stage, items = (m-tile, n-tile)

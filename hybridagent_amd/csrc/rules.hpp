@@ -1,5 +1,6 @@
-// Which kernel a call's bf16 linears run: host rules on sizes alone, free of
-// HIP so that they can be checked without a GPU.
+// Which kernel a call's bf16 linears run, and the height of the tiled GEMMs'
+// tiles: host rules on sizes alone, free of HIP so that they can be checked
+// without a GPU.
 #pragma once
 #include <stdint.h>
 
@@ -33,6 +34,44 @@ inline bool linear_tiled_rows(int64_t M, int64_t N, int64_t K) {
 // they are held.
 inline bool ffn_fragment_rows(int64_t M, int64_t H, int64_t Im, bool fits, bool tiles_supported) {
   return M > 16 && fits && !(tiles_supported && linear_tiled_frag(M, Im, H));
+}
+
+// The tile height, in 32-row blocks, of a launch whose tiles (256 weight rows
+// each) are all alike and run one per CU: the time is the rounds of tiles times
+// a tile's, cost[blocks - 1].
+inline int cheapest_blocks(int64_t M, int64_t wrows, int cus, int max_blocks, const int* cost) {
+  const int64_t n_nt = (wrows + 255) / 256;
+  int best = 0;
+  int64_t least = 0;
+  for (int mb = 1; mb <= max_blocks; ++mb) {
+    const int64_t tiles = (M + 32 * mb - 1) / (32 * mb) * n_nt;
+    const int64_t c = (tiles + cus - 1) / cus * cost[mb - 1];
+    if (best == 0 || c < least) {
+      best = mb;
+      least = c;
+    }
+  }
+  return best;
+}
+
+// Dense bf16 GEMM: a tile's time is close to (blocks + 1), its MFMAs and a
+// stage's weights, barrier and waits whatever the height.  The FFN block (Im =
+// 2112, flat routing) with 1 .. 5 blocks: 287 / 265 / 270 / 283 / 288 us at 512
+// rows (2 picked), 399 / 354 / 336 / 346 / 353 at 1024 (3), 572 / 521 / 480 /
+// 490 / 468 at 2048 (gate/up 5, down 3: 464).
+constexpr int kGemmMaxBlocks = 5;
+inline int gemm_bf16_blocks(int64_t M, int64_t wrows, int cus) {
+  constexpr int cost[kGemmMaxBlocks] = {2, 3, 4, 5, 6};
+  return cheapest_blocks(M, wrows, cus, kGemmMaxBlocks, cost);
+}
+
+// Linear4Bit tiles of at most max_blocks: a tile of 1 .. 6 blocks measured 24,
+// 27, 33, 34, 41, 48 us at K = 2816 (a stage's barrier and waits dominate few
+// blocks).
+constexpr int kLinearW4MaxBlocks = 6;
+inline int linear_w4_blocks(int64_t M, int64_t N, int cus, int max_blocks) {
+  constexpr int cost[kLinearW4MaxBlocks] = {24, 27, 33, 34, 41, 48};
+  return cheapest_blocks(M, N, cus, max_blocks, cost);
 }
 
 }  // namespace w4a16

@@ -1,5 +1,6 @@
-"""The host rules that choose a call's bf16 linears, compiled for the CPU: the
-lines measured on an MI355X, and that every call has exactly one kernel."""
+"""The host rules that choose a call's bf16 linears and the tiles' heights, compiled
+for the CPU: the lines measured on an MI355X, that every call has exactly one
+kernel, and that the heights follow the number of CUs."""
 import shutil
 import subprocess
 from pathlib import Path
@@ -18,6 +19,8 @@ int main() {
   while (scanf("%15s %lld %lld %lld %lld", what, &a, &b, &c, &d) == 5) {
     if (what[0] == 'f') printf("%d\\n", (int)ffn_fragment_rows(a, b, c, d & 1, d & 2));
     else if (what[0] == 'r') printf("%d\\n", (int)linear_tiled_rows(a, b, c));
+    else if (what[0] == 'g') printf("%d\\n", gemm_bf16_blocks(a, b, c));
+    else if (what[0] == 'l') printf("%d\\n", linear_w4_blocks(a, b, c, d));
     else return 1;
   }
 }
@@ -65,3 +68,20 @@ def test_no_call_of_many_rows_streams_row_major(ask):
     frag = ask([("f", M, K, N, 3) for M, K, N in sizes])
     tiled = ask([("r", M, N, K, 0) for M, K, N in sizes])
     assert all(f or t for f, t in zip(frag, tiled))
+
+
+def test_tile_heights_at_256_cus(ask):
+    # the FFN block's gate/up (4224 weight rows) and down, Linear4Bit at 2816 x 2816
+    assert ask([("g", 512, 4224, 256, 0), ("g", 1024, 4224, 256, 0), ("g", 2048, 4224, 256, 0),
+                ("g", 2048, 2816, 256, 0), ("l", 2048, 2816, 256, 6), ("l", 4096, 2816, 256, 6),
+                ("l", 4096, 2816, 256, 4)]) == [2, 3, 5, 3, 3, 6, 3]
+
+
+@pytest.mark.parametrize("cus", [32, 64, 128, 256, 304])
+def test_tile_heights_are_the_cheapest_for_the_cus(ask, cus):
+    gemm, w4 = [2, 3, 4, 5, 6], [24, 27, 33, 34, 41, 48]
+    sizes = [(M, n) for M in (65, 300, 1024, 2048, 4096) for n in (704, 2816, 4224)]
+    got = ask([("g", M, n, cus, 0) for M, n in sizes] + [("l", M, n, cus, 6) for M, n in sizes])
+    for (M, n), cost, mb in zip(sizes * 2, [gemm] * len(sizes) + [w4] * len(sizes), got):
+        time = [-(-(-(-M // (32 * b)) * -(-n // 256)) // cus) * c for b, c in enumerate(cost, 1)]
+        assert time[mb - 1] == min(time), (M, n, mb, time)
