@@ -87,6 +87,28 @@ def test_bf16_experts_streamed_segments(dev, rows):
             assert ((got[t] - ref).abs() <= slack).all(), f"expert {e} of {rows[e]} rows"
 
 
+# routed rows that are no multiple of four, all of them valid: the last row indices come in a 16-byte load that is
+# partly past the plan's
+@pytest.mark.parametrize("M,k", [(193, 1), (194, 1), (195, 1), (65, 3), (66, 3), (67, 3)])
+def test_bf16_experts_last_rows(dev, M, k):
+    E, H, I = 4, 256, 192
+    g = torch.Generator(device=dev).manual_seed(61)
+    gu = (torch.randn(E, 2 * I, H, generator=g, device=dev) / math.sqrt(H)).to(torch.bfloat16)
+    dn = (torch.randn(E, H, I, generator=g, device=dev) / math.sqrt(I)).to(torch.bfloat16)
+    gc = torch.Generator().manual_seed(62)
+    idx = torch.stack([torch.randperm(E, generator=gc)[:k] for _ in range(M)])
+    x = synth.activations(M, H, seed=63, device=dev)
+    # one slot's weight at a time, so that every routed row of the last expert's segment shows
+    for j in range(k):
+        w = torch.zeros(M, k, device=dev)
+        w[:, j] = 1.0
+        got = _lib.bf16_experts_forward(x, idx.to(dev), w, gu, dn).double()
+        for e in range(E):
+            t = (idx[:, j] == e).nonzero()[:, 0].to(dev)
+            ref, slack = _mlp64(x[t].double(), gu[e, :I].double(), gu[e, I:].double(), dn[e].double())
+            assert ((got[t] - ref).abs() <= slack).all(), f"expert {e}, slot {j}"
+
+
 @pytest.mark.parametrize("H,I", [(256, 192), (160, 160)])
 def test_bf16_experts_two_slots_and_invalid(dev, H, I):
     # token-slot gathers (row / top_k) and slots without an expert, against the same routing on fp64

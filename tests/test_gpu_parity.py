@@ -483,31 +483,33 @@ def test_moe_prefill_half_items(dev, h, i, G):
 
 @pytest.mark.parametrize("h,i,G", [(1024, 704, 128), (896, 960, 256)])
 def test_moe_prefill_wide_items_bit_identical(dev, h, i, G):
-    # an expert's tail of at most 32 rows runs as a wide item (three n-tiles
-    # per workgroup item), of more rows as a one-n-tile item: the same token
-    # rows give the same bits either way.  Batch A: expert 0 holds 20 rows
-    # (wide); batch B = A + 20 tokens on experts 0 and 7: expert 0 holds 40
-    # rows (one-n-tile item of two m-blocks)
-    e, k = 8, 2
+    # on the tiled weights, where every segment is at most 32 rows, the
+    # segments run as wide items (three n-tiles per workgroup item), among
+    # larger segments as one-n-tile items: the same token rows give the same
+    # bits either way.  Batch A: 24 experts of 2 .. 32 rows (wide); batch B =
+    # A + 40 tokens on experts 0 and 7, 72 and 65 rows (no wide items)
+    e, k = 24, 2
     wts = synth.moe_weights(e, h, i, G, seed=790)
-    counts = [20, 180, 100, 60, 33, 30, 97, 80]
+    counts = [32, 31, 30, 2, 20, 32, 16, 25] * 3
     M = sum(counts) // k
     slots = np.repeat(np.arange(e), counts)
     idx = np.stack([slots[:M], slots[M:]], 1)
     assert (idx[:, 0] != idx[:, 1]).all()
     idx = idx[np.random.default_rng(791).permutation(M)]
-    extra = np.tile(np.array([[0, 7]]), (20, 1))
+    extra = np.tile(np.array([[0, 7]]), (40, 1))
     idx_b = torch.from_numpy(np.concatenate([idx, extra])).long()
-    x_b = synth.activations(M + 20, h, seed=792)
-    w_b = torch.rand(M + 20, k, generator=torch.Generator().manual_seed(793)).float()
+    assert M > 256 and max(counts) <= 32 and int(torch.bincount(idx_b.flatten()).max()) == 72
+    x_b = synth.activations(M + 40, h, seed=792)
+    w_b = torch.rand(M + 40, k, generator=torch.Generator().manual_seed(793)).float()
     gpu = [wts.gate_up_packed.to(dev), wts.gate_up_scale.to(dev), wts.down_packed.to(dev), wts.down_scale.to(dev)]
-    print(f"prefill wide items h={h} i={i} G={G} M={M} / {M + 20}", flush=True)
-    y_a = _lib.moe_forward(x_b[:M].to(dev), idx_b[:M].to(dev), w_b[:M].to(dev), *gpu).cpu()
-    y_b = _lib.moe_forward(x_b.to(dev), idx_b.to(dev), w_b.to(dev), *gpu).cpu()
+    tiles = _lib.tile_experts(*gpu, G)
+    print(f"prefill wide items h={h} i={i} G={G} M={M} / {M + 40}", flush=True)
+    y_a = _lib.moe_forward(x_b[:M].to(dev), idx_b[:M].to(dev), w_b[:M].to(dev), *gpu, G, tiles=tiles).cpu()
+    y_b = _lib.moe_forward(x_b.to(dev), idx_b.to(dev), w_b.to(dev), *gpu, G, tiles=tiles).cpu()
     assert torch.equal(y_a, y_b[:M])
     ref = oracle.moe_forward(_np(x_b), idx_b.numpy(), w_b.numpy(), wts.gate_up_packed.numpy(),
                              _bits(wts.gate_up_scale), wts.down_packed.numpy(), _bits(wts.down_scale), G)
-    assert margin(f"moe prefill wide items h={h} i={i} G={G} M={M + 20} (all rows)",
+    assert margin(f"moe prefill wide items h={h} i={i} G={G} M={M + 40} (all rows)",
                   oracle.max_abs_rel(_np(y_b), ref)) <= TOL
 
 

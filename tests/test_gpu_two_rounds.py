@@ -3,7 +3,7 @@ chip's workgroups, at most two thirds): a token's row equals, bit for bit, the
 same token's in calls of 32 tokens, which run one round -- on a plan the sort
 wrote (moe_forward) and on the launch's own (moe_layer_forward at M * top_k
 <= 1024), packed and tiled, either side of the slot range, whose slot count the
-routing is made to hit."""
+routing is made to hit on both."""
 import pytest
 import torch
 
@@ -52,22 +52,29 @@ def test_two_rounds_bit_identical(M, n_full, slots, G, tiled):
         assert torch.equal(_lib.moe_forward(x[s], idx[s], wt[s], *ew, G, tiles=tiles), y[s]), f"rows {m}.."
 
 
-@pytest.mark.parametrize("M", [112, 121, 128])
+@pytest.mark.parametrize("M,n_full,slots", [(112, 0, 128), (112, 1, 129), (121, 20, 148), (128, 42, 170),
+                                            (128, 43, 171)])
 @pytest.mark.parametrize("tiled", [False, True])
-def test_two_rounds_own_plan(M, tiled):
-    # skewed routing: more than 128 slots among M * top_k <= 1024 rows
+def test_two_rounds_own_plan(M, n_full, slots, tiled):
+    # the launch plans for itself (896 <= M * top_k <= 1024); the router's rows make it choose this routing
     dev = torch.device("cuda:0")
     G = 128
     w = synth.moe_weights(E, H, I, G, seed=91, device=dev)
     ew = (w.gate_up_packed, w.gate_up_scale, w.down_packed, w.down_scale)
     tiles = _lib.tile_experts(*ew, G) if tiled else None
-    for beta in (0.3, 0.6, 1.0):
-        rw = synth.zipf_router_weights(E, H, seed=92, s=1.1, beta=beta, n_empty=0, device=dev)
-        x = synth.zipf_activations(M, H, seed=93, device=dev)
-        out, wt, idx = _lib.moe_layer_forward(x, rw.scale, rw.scalar_root, rw.proj, rw.per_expert_scale, rw.eps, K, x,
-                                              *ew, G, tiles=tiles)
-        slots = int(((torch.bincount(idx.flatten(), minlength=E) + 15) // 16).sum())
-        print(f"own plan M={M} beta={beta} slots={slots} tiled={tiled}", flush=True)
-        for m in range(0, M, 32):
-            s = slice(m, m + 32)
-            assert torch.equal(_lib.moe_forward(x[s], idx[s], wt[s], *ew, G, tiles=tiles), out[s]), f"rows {m}.."
+    want, n = _routing(M, n_full, 92)
+    assert n == slots
+    # expert e's router weights are coordinate e, a row's coordinates its experts' scores, best first
+    proj = torch.zeros(E, H, dtype=torch.bfloat16)
+    proj[torch.arange(E), torch.arange(E)] = 1.0
+    rows = torch.zeros(M, H).scatter_(1, want, torch.linspace(8.0, 4.5, K).expand(M, K).contiguous())
+    x = synth.activations(M, H, seed=93, device=dev)
+    one = torch.ones(H, dtype=torch.bfloat16, device=dev)
+    pes = torch.ones(E, dtype=torch.bfloat16, device=dev)
+    print(f"own plan M={M} slots={slots} tiled={tiled}", flush=True)
+    out, wt, idx = _lib.moe_layer_forward(rows.to(torch.bfloat16).to(dev), one, 1.0, proj.to(dev), pes, 1e-6, K, x,
+                                          *ew, G, tiles=tiles)
+    assert torch.equal(idx.cpu(), want)
+    for m in range(0, M, 32):
+        s = slice(m, m + 32)
+        assert torch.equal(_lib.moe_forward(x[s], idx[s], wt[s], *ew, G, tiles=tiles), out[s]), f"rows {m}.."
