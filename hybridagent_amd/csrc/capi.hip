@@ -91,9 +91,15 @@ inline bool linear_w4_tiled(int64_t M, int64_t N) { return M > 64 && M * N > 900
 
 // The BF16 experts' routed rows up to which their weights stream once per
 // 16..64 rows of an expert (k_bf16_expert); above, the tiled GEMM (an
-// expert's weights once per 128 rows).  Gemma shape at 128 / 256 / 512 / 8248
-// rows: 192 / 267 / 315 / 1341 us streamed, 178 / 243 / 271 / 329 us tiled;
-// with Zipf-skewed routing 135 / 202 / 335 us against 142 / 158 / 231.
+// expert's weights once per 128 rows).  What decides is the rows per expert
+// hit and the bytes of an expert; the line is where 128 experts of the Gemma
+// shape cross, at 128 / 256 / 512 / 8248 rows 204 / 269 / 314 / 1316 us
+// streamed, 202 / 245 / 270 / 332 tiled (flat routing) and 142 / 217 / 304 /
+// 1510 .. 1860 against 149 / 182 / 233 / 380 (Zipf 1.1).  Above it the tiles
+// were faster at every other count measured too: at 256 rows 8 experts top-2
+// 83 / 45, 32 experts 73 / 44, 64 169 / 155, 256 256 / 212, 512 120 / 73 us
+// (flat; the skewed ones alike).  At most of those counts they would be faster
+// below it as well: 512 experts at 64 rows 45 / 33, 8 experts at 128 70 / 41.
 constexpr int64_t kBf16StreamMaxRows = 192;
 
 // The FFN block's last launch (launch_ffn_post), run by the layer in place of
@@ -1052,9 +1058,10 @@ int moe_bf16_experts_forward(const uint16_t* hidden, const int64_t* topk_idx, co
                               L.counters, L.tiles, L.blockcnt, kPrefillBM, 0, s, L.queues)
           : launch_sort(topk_idx, (int)M, (int)top_k, (int)E, L.sorted_pos, L.offsets, L.desc,
                         L.counters, L.tiles, kPrefillBM, 0, s, L.queues);
-  // the tile list holds an expert's tile index in 16 bits
-  if (M * top_k > kBf16StreamMaxRows && M * top_k <= int64_t(65535) * kPrefillBM && gemm_bf16_supported(H, I) &&
-      gemm_bf16_supported(I, H)) {
+  // (the tile list holds an expert's tile index in 16 bits: M top_k <= 2^30 /
+  // max(H, I), and the GEMM takes H, I >= 160, so an expert has at most 52,429
+  // tiles of 128 rows)
+  if (M * top_k > kBf16StreamMaxRows && gemm_bf16_supported(H, I) && gemm_bf16_supported(I, H)) {
     GemmBf16Args g{};
     g.sorted_pos = L.sorted_pos;
     g.offsets = L.offsets;

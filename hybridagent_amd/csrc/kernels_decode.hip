@@ -915,6 +915,10 @@ static hipError_t launch_stream(DecodeArgs a, int ncolblk, int max_slots, hipStr
   // it likely.  The workgroups it does not need leave at once, in kSelfPlan
   // after their own plan: 96 tokens x top-8 (128 slots) 108 us with and
   // without them, 96 tokens of skewed routing (145 slots) 144 -> 126 us.
+  // Measured at 128 experts top-8; with the same line, before and with two
+  // rounds, at G = 32: 64 experts top-8, 193 / 256 tokens 101 / 94, 143 / 126;
+  // 128 top-4, 256 tokens (G = 128) 142 / 125; 256 and 512 experts, which have
+  // more slots than the rule takes, unchanged.
   constexpr int64_t kTwoRoundRows = SELF == kSelfPlan ? 896 : 768;
   a.resident = 0;
   if (two_rounds<MODE, KSPLIT, SELF>() && !narrow && per_cu == 1 &&

@@ -52,10 +52,14 @@
 // chain over all of K the FFN block at 2048 rows takes 492.8 us, not 490.4,
 // and 1031 tokens of BF16 experts 380.5, not 379.5.
 //
-// Bound: the experts by their weights' stream (1031 tokens x top-8, 128
-// experts of 11.9 MB: 1.64 ms streamed per 64 rows, 0.38 ms here, 4.1 TB/s
-// over the layer); the dense form by LDS reads and the stage barrier (shared
-// MLP of 2048 rows, 73 GFLOP: 830 us -> 97 us).
+// Bound: the experts by their weights' stream (1031 tokens x top-8 over 128
+// experts of 11.9 MB, flat routing: the call 1316 us streamed per 64 rows, 332
+// here, 4.6 TB/s; skewed, Zipf 1.1: 1510 .. 1860 and 380).  The dense form by
+// no one unit: gate/up of 2048 rows x 2 x 2112 (58 us, five blocks) has the
+// MFMAs busy 35 % of the time and LDS 21 %, without bank conflicts; its
+// wavefronts wait for loads and at the stage barrier for 30 % of theirs and to
+// issue for 31 % (shared MLP of 2048 rows, 73 GFLOP: 830 us streamed, about 95
+// here).
 #include <type_traits>
 
 #include "common.hpp"

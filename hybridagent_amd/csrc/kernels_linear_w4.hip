@@ -19,8 +19,10 @@
 // stage (K % 64 == 32) has only h = 0's, so the lanes of h = 1 multiply zeros
 // there and their loads are turned to the row's bytes before.
 //
-// Bound: the dequantisation's VALU beside the MFMAs, and the last round of
-// tiles.  2816 x 2816, G = 32, at 512 / 1024 / 2048 / 4096 rows:
+// Bound: no one unit.  2816 x 2816 at 2048 rows (three blocks, 242 tiles, one
+// round): 7.8 VALU per MFMA, issued for 34 % of the time, the MFMAs busy for 30
+// %, LDS for 21 %; the wavefronts wait for loads and at the stage barrier for
+// 40 % of theirs.  2816 x 2816, G = 32, at 512 / 1024 / 2048 / 4096 rows:
 // streamed 33 / 54 / 99 / 186 us, here 24 / 28 / 40 / 64 us (815 TFLOP/s at 2048).
 #include <type_traits>
 

@@ -13,8 +13,8 @@
 // with all their n-tiles and a queue of its own; gate_up has one queue for
 // the chip.  Each of the eight wavefronts owns 32
 // weight rows (gate_up: 16 gate + their 16 up rows) for all the item's
-// rows: MB m-blocks of v_mfma_f32_32x32x16_bf16 accumulators (MB = 8 for
-// 256 rows; 4, 2, 1 for segment tails of up to 128, 64, 32 rows).
+// rows: MB m-blocks of v_mfma_f32_32x32x16_bf16 accumulators, MB = the item's
+// 32-row blocks, 1 .. 8 (gate_up's half n-tile: 1 .. 4 per wavefront half).
 //
 // The small tails (most of them are whole experts of few rows) give a stage
 // little MFMA work, so what a stage costs whatever its rows decides.
@@ -999,7 +999,9 @@ __device__ __forceinline__ int px_dispatch(const PrefillArgs& a, unsigned char* 
 // differ more in cost (segment tails, the half n-tile) and the XCDs in
 // speed, and the whole chip draining one queue ends them closer together
 // than the rows kept in one L2 save.  The list runs from large tiles to
-// small, so large items go first.  Workgroups ask in the order they get
+// small but for the tails of at most kPrefillTinyRows rows, which stand before
+// the other tails: as wide items they are the longer ones and are taken there,
+// as tail items last (px_item_info).  Workgroups ask in the order they get
 // there, during the last stage of the item before their next one, so the
 // index is known one item ahead (the next item's rows and first stages are
 // loaded during the current one).  queues[8] counts the workgroups that

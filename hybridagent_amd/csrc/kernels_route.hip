@@ -624,9 +624,11 @@ hipError_t launch_router_topk(const float* partial, int ksplit, const uint16_t* 
 //   tiles[i] = (expert << 16) | m_tile for the i-th (expert, m-tile) pair:
 //     first every tile of more than BM / 2 rows, then the segment tails of at
 //     most kPrefillTinyRows rows, then the other tails of at most BM / 2 rows
-//     (expert order each).  Work queues hand tiles out in list order, and the
-//     prefill GEMM takes the smallest tails three n-tiles at a time, which
-//     makes those items longer than the other tails'.
+//     (expert order each).  Work queues hand tiles out in list order; the
+//     exact-form prefill GEMM takes the smallest tails where they stand when
+//     it takes three n-tiles of each at a time (tiled weights, nearly all
+//     m-tiles such tails), which makes those items the longer ones, and last
+//     otherwise.
 // ---------------------------------------------------------------------------
 constexpr int kSortThreads = 1024;
 constexpr int kSortWaves = kSortThreads / 64;

@@ -16,7 +16,8 @@ constexpr int kPfBN = 128;
 // m-tile of the exact-form prefill GEMM (kernels_prefill_x.hip)
 constexpr int kPrefillXBM = 256;
 // segment tails of at most this many rows (one 32-row MFMA block) are listed
-// apart, and the exact-form prefill GEMM takes them three n-tiles per item
+// apart: on the tiled weights, where nearly all m-tiles are such tails, the
+// exact-form prefill GEMM takes them three n-tiles per item, else last
 constexpr int kPrefillTinyRows = 32;
 // prefill work-queue counters in the MoE workspace: gate_up [0, 16), down [16, 32)
 constexpr int kPrefillQueueInts = 32;
