@@ -41,7 +41,8 @@ def test_bf16_experts_rows(dev, H, I):
 
 
 @pytest.mark.parametrize("H,Im,M", [(288, 2112, 1411), (2816, 1056, 300), (2816, 2112, 129), (2816, 2112, 481),
-                                    (2816, 1120, 1025), (2816, 2112, 2048)])
+                                    (2816, 1120, 1025), (2816, 2112, 2048), (2816, 352, 2300),
+                                    (2816, 352, 3000)])
 def test_ffn_shared_mlp_rows(dev, H, Im, M):
     """The block with experts whose weights are all zero (q = 0): its output is norm3(norm1(mlp) + 0)."""
     I, E, G = 192, 4, 32

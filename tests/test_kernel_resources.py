@@ -3,11 +3,11 @@ direct loads in flight across their epilogue spill no vector register (a reload
 there waits for every load and store in flight)."""
 import struct
 
-import msgpack
 import pytest
 
 from hybridagent_amd.build import LIB_PATH
 
+msgpack = pytest.importorskip("msgpack")
 MAGIC = b"__CLANG_OFFLOAD_BUNDLE__"
 
 
