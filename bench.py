@@ -53,6 +53,7 @@ rotated through HBM).
 from __future__ import annotations
 
 import argparse
+import gc
 import json
 import math
 import os
@@ -156,13 +157,20 @@ def time_dispatches(fns, reps: int, warmup: int = 1) -> float:
             f()
     torch.cuda.synchronize()
     pairs = []
-    for _ in range(reps):
-        for f in fns:
-            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-            a.record()
-            f()
-            b.record()
-            pairs.append((a, b))
+    # a garbage collection between a pair's first event and its launch would be
+    # counted as the launch's time
+    gc.collect()
+    gc.disable()
+    try:
+        for _ in range(reps):
+            for f in fns:
+                a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+                a.record()
+                f()
+                b.record()
+                pairs.append((a, b))
+    finally:
+        gc.enable()
     torch.cuda.synchronize()
     return sum(a.elapsed_time(b) for a, b in pairs) * 1e-3 / len(pairs)
 
