@@ -83,10 +83,11 @@ struct AddNorm {
 
 // Whether Linear4Bit (M rows, N columns) runs as the tiled GEMM instead of
 // streaming its weights once per 16 rows (k_decode<dense>).  Few tiles take a
-// tile's time, which grows with K as the stream's does.  K = 2816, streamed /
-// tiled, in us: N = 2816 at 256 / 384 / 2048 rows 21/24, 30/24, 99/40 (G = 32;
-// 20/25, 27/26, 90/40 at G = 128); N = 1408 at 512 / 768 rows 21/24, 30/24;
-// K = 1056, N = 704 at 1024 / 1536 rows 16/16, 21/16.
+// tile's time, which grows with K as the stream's does.  Either side of the
+// line, streamed / tiled, in us: K = 2816, N = 2816, 319 / 320 rows 25/26 (G =
+// 32), 23/25 (G = 128), N = 1408, 639 / 640 rows 26/26; K = 1056, N = 704, 1278
+// / 1279 rows 17/13; K = 704, N = 2816, 319 / 320 rows 10.4/9.8; far above it
+// 2048 rows of 2816 x 2816 99/41.
 inline bool linear_w4_tiled(int64_t M, int64_t N) { return M > 64 && M * N > 900000; }
 
 // The BF16 experts' routed rows up to which their weights stream once per

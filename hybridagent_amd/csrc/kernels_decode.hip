@@ -21,6 +21,7 @@
 
 #include "common.hpp"
 #include "launch.hpp"
+#include "rules.hpp"
 #include "route_device.hpp"
 
 namespace w4a16 {
@@ -791,22 +792,6 @@ void k_decode(DecodeArgs a) {
   }
 }
 
-// Decode launch shapes: (k tiles per wavefront, wavefronts per K range).
-struct DecodeShape {
-  int tpw;
-  int ksplit;
-};
-
-static DecodeShape decode_shape(int K) {
-  const int ntiles = ((K >> 5) + 3) >> 2;
-  if (ntiles <= 2) return {2, 1};
-  if (ntiles <= 4) return {4, 1};
-  if (ntiles <= 6) return {6, 1};   // down, K = 704: 6 tiles, 4 column groups
-  if (ntiles <= 8) return {2, 4};
-  if (ntiles <= 16) return {4, 4};
-  return {6, 4};                    // gate_up, K = 2816: 22 tiles over 4 wavefronts
-}
-
 // activation rows staged per LDS pass: the largest power of two <= 16 whose
 // fragment-layout footprint fits the shape's LDS budget
 static int stage_rows(int K, int ksplit) {
@@ -957,7 +942,7 @@ static hipError_t launch_decode_mode(DecodeArgs a, int max_slots, hipStream_t s)
 #define W4A16_DEC(T_, K_)                                                          \
   return wide ? launch_stream<MODE, T_, K_, false, true>(a, ncolblk, max_slots, s) \
               : launch_stream<MODE, T_, K_, false, false>(a, ncolblk, max_slots, s)
-  if (ntiles > 24) return launch_stream<MODE, 6, 4, true>(a, ncolblk, max_slots, s);
+  if (decode_ranges_interleave(a.K)) return launch_stream<MODE, 6, 4, true>(a, ncolblk, max_slots, s);
   if (sh.ksplit == 1) {
     if (sh.tpw == 2) W4A16_DEC(2, 1);
     if (sh.tpw == 4) W4A16_DEC(4, 1);

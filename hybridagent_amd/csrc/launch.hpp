@@ -300,7 +300,7 @@ hipError_t launch_ffn_post(const FfnPostCall& c, const uint16_t* moe, const int6
 // BF16 experts: grid (column tile, active slot), max_slots <= 65535
 hipError_t launch_bf16_experts(int mode, Bf16ExpertArgs a, int max_slots, hipStream_t s);
 // Linear4Bit at prefill sizes (kernels_linear_w4.hip): K a multiple of 32
-// above 128 whose scales fit in LDS
+// above 128 (of 128 above 3072) whose scales fit in LDS
 bool linear_w4_supported(int64_t K, int64_t G);
 hipError_t launch_linear_w4(const uint16_t* x, const int32_t* wp, const uint16_t* ws, const uint16_t* bias,
                             uint16_t* y, int64_t M, int64_t N, int64_t K, int64_t G, hipStream_t s);

@@ -65,12 +65,35 @@ inline int gemm_bf16_blocks(int64_t M, int64_t wrows, int cus) {
   return cheapest_blocks(M, wrows, cus, kGemmMaxBlocks, cost);
 }
 
-// Linear4Bit tiles of at most max_blocks: a tile of 1 .. 6 blocks measured 24,
-// 27, 33, 34, 41, 48 us at K = 2816 (a stage's barrier and waits dominate few
-// blocks).
+// The decode streamer's shape for K: k tiles (128 wide) per wavefront in a row
+// and wavefronts per sum.  It is also what a sum is: wavefront w's fp32 chain
+// over the tiles w tpw .. w tpw + tpw - 1, and those a multiple of ksplit tpw
+// behind them, the wavefronts' chains added in order.
+struct DecodeShape {
+  int tpw;
+  int ksplit;
+};
+inline DecodeShape decode_shape(int64_t K) {
+  const int64_t ntiles = (K + 127) / 128;
+  if (ntiles <= 2) return {2, 1};
+  if (ntiles <= 4) return {4, 1};
+  if (ntiles <= 6) return {6, 1};   // down, K = 704: 6 tiles, 4 column groups
+  if (ntiles <= 8) return {2, 4};
+  if (ntiles <= 16) return {4, 4};
+  return {6, 4};                    // gate_up, K = 2816: 22 tiles over 4 wavefronts
+}
+// whether a chain's tiles lie apart (more than ksplit tpw tiles)
+inline bool decode_ranges_interleave(int64_t K) {
+  const DecodeShape s = decode_shape(K);
+  return (K + 127) / 128 > s.tpw * s.ksplit;
+}
+
+// Linear4Bit tiles of at most max_blocks: one round of tiles of 1 .. 6 blocks
+// measured 31, 37, 44, 52, 61, 72 us at K = 2816, 11.0 .. 25.4 at K = 704 (a
+// stage's barrier and waits dominate few blocks).
 constexpr int kLinearW4MaxBlocks = 6;
 inline int linear_w4_blocks(int64_t M, int64_t N, int cus, int max_blocks) {
-  constexpr int cost[kLinearW4MaxBlocks] = {24, 27, 33, 34, 41, 48};
+  constexpr int cost[kLinearW4MaxBlocks] = {31, 37, 44, 52, 61, 72};
   return cheapest_blocks(M, N, cus, max_blocks, cost);
 }
 

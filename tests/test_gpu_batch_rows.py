@@ -1,8 +1,8 @@
-"""A row's bits do not depend on the batch around it where the bf16 weights are
-concerned: the BF16 experts and the FFN block's shared MLP sum every output over
-the same ranges of K in the same order, whether a call streams the weights (few
-rows) or runs the tiled GEMM (many).  Every row of a large call is compared with
-the same row in calls of few rows, bit for bit.
+"""A row's bits do not depend on the batch around it: the BF16 experts, the FFN
+block's shared MLP and Linear4Bit sum every output over the same ranges of K in
+the same order, whether a call streams the weights (few rows) or runs the tiled
+GEMM (many).  Rows of a large call are compared with the same rows in calls of
+few rows, bit for bit.
 
 The shapes: ranges of one 32-wide step (K <= 256), ranges that end inside a
 64-wide stage, K ranges without a step (K / 32 not filling them), a last half
@@ -64,3 +64,17 @@ def test_ffn_shared_mlp_rows(dev, H, Im, M):
     # 64 rows stream the weights on fragment-order rows, 16 on row-major ones
     for lo, n in [(0, 64), (M // 2, 64), (M - 64, 64), (M - 16, 16), (M - 1, 1)]:
         assert torch.equal(whole[lo:lo + n], block(slice(lo, lo + n))), f"rows from {lo}"
+
+
+# K: one to four ranges of every length, a range without a tile (2112), tiles of 1 to 4 32-wide chunks last, ranges
+# whose tiles lie apart (3200, 9216); M at N = 2816: every tile height, 1 .. 6 row blocks, whole and not
+@pytest.mark.parametrize("K", [160, 256, 352, 512, 672, 704, 992, 1056, 2048, 2112, 2816, 3072, 3200, 9216])
+@pytest.mark.parametrize("M,N,G", [(330, 2816, 32), (700, 2816, 128), (1201, 2816, 32), (1800, 2816, 64),
+                                   (2300, 2816, 32), (4096, 2816, 128), (700, 1357, 32)])
+def test_linear4bit_rows(dev, K, M, N, G):
+    p = synth.packed_int4((N, K), 61, dev)
+    s = synth.group_scales((N, K), G, 62, dev)
+    x = synth.activations(M, K, 63, dev)
+    whole = _lib.linear(x, p, s, None, G)
+    for lo, n in [(0, 300), (M // 2, 17), (M - 300, 300), (M - 1, 1)]:  # at most 900e3 outputs stream the weights
+        assert torch.equal(whole[lo:lo + n], _lib.linear(x[lo:lo + n], p, s, None, G)), f"rows from {lo}"

@@ -79,7 +79,7 @@ def test_tile_heights_at_256_cus(ask):
 
 @pytest.mark.parametrize("cus", [32, 64, 128, 256, 304])
 def test_tile_heights_are_the_cheapest_for_the_cus(ask, cus):
-    gemm, w4 = [2, 3, 4, 5, 6], [24, 27, 33, 34, 41, 48]
+    gemm, w4 = [2, 3, 4, 5, 6], [31, 37, 44, 52, 61, 72]
     sizes = [(M, n) for M in (65, 300, 1024, 2048, 4096) for n in (704, 2816, 4224)]
     got = ask([("g", M, n, cus, 0) for M, n in sizes] + [("l", M, n, cus, 6) for M, n in sizes])
     for (M, n), cost, mb in zip(sizes * 2, [gemm] * len(sizes) + [w4] * len(sizes), got):
