@@ -142,36 +142,36 @@ constexpr int kSelfMaxExperts = 128;
 constexpr int kSortWavesMax = 16;  // wavefronts of the wide form
 
 // Workgroups per slot for U active slots and `grid` workgroups: as many as
-// fit on the chip at once (a.resident; 0: the whole grid).  Between a half
+// fit on the chip at once (TWO: a.resident, fewer than the grid).  Between a half
 // and two thirds of that many slots one each would leave up to half of the
 // chip idle while the others walk a whole expert; three each, in two rounds,
 // walk two thirds of one, a second stage included (193 tokens x top-8 at the
 // Gemma shape, G = 32, about 140 slots: the layer 149 -> 134 us tiled, 184 ->
-// 161 us packed; 128 tokens 146 -> 130 us).  Compiled in only where the
-// launcher may ask for it (two_rounds): its scalar work comes before a slot's
-// first load (a dense 2816 x 704 call of 4 rows 5.1 us with it, 4.8 without).
+// 161 us packed; 128 tokens 146 -> 130 us).  A kernel of its own (TWO), for the
+// forms that may ask for it (two_rounds): its scalar work comes before a
+// slot's first load (a dense 2816 x 704 call of 4 rows 5.1 us with it, 4.8
+// without; layers of 16 tokens, G = 32, 84.8 and 84.4).
 template <int MODE, int KSPLIT, int SELF>
 constexpr bool two_rounds() {
   return MODE == kModeGateUp && KSPLIT == 4 && SELF != kSelfRoute;
 }
 template <bool TWO>
 __host__ __device__ __forceinline__ int slot_wgs(const DecodeArgs& a, int U, int grid) {
-  if (!TWO) {
-    const int n = grid / U;
-    return n < 1 ? 1 : n < a.n_ct ? n : a.n_ct;
+  if (TWO) {
+    if (2 * U > a.resident && 3 * U <= grid && 3 * U <= 2 * a.resident) return a.n_ct < 3 ? a.n_ct : 3;
+    grid = a.resident > U ? a.resident : U;
   }
-  if (a.resident > 0 && 2 * U > a.resident && 3 * U <= grid && 3 * U <= 2 * a.resident) return a.n_ct < 3 ? a.n_ct : 3;
-  const int n = (a.resident > 0 && a.resident < grid ? (a.resident > U ? a.resident : U) : grid) / U;
-  return n < 1 ? 1 : n < a.n_ct ? n : a.n_ct;
+  const int n = grid / U < a.n_ct ? grid / U : a.n_ct;
+  return n > 1 ? n : 1;
 }
 
 template <int MODE, int TPW, int KSPLIT, bool LONGK, bool WIDE, bool TILED = false, bool LSCALE = false,
-          int SELF = kSelfNone>
+          int SELF = kSelfNone, bool TWO = false>
 __global__ __launch_bounds__(stream_threads(KSPLIT)) __attribute__((amdgpu_waves_per_eu(TPW >= 4 ? 2 : 4, 8)))
 void k_decode(DecodeArgs a) {
   constexpr int kStreamThreads = stream_threads(KSPLIT);  // the wide form
   constexpr int NWAVES = kStreamThreads / 64;
-  constexpr bool kTwo = two_rounds<MODE, KSPLIT, SELF>();
+  static_assert(!TWO || two_rounds<MODE, KSPLIT, SELF>(), "two rounds of gate_up");
   const int CG = a.cg;  // column groups per item: 4 (wide) or 1 (narrow)
   extern __shared__ __align__(16) unsigned char smem_raw[];
   u32x4_t* __restrict__ lds_a = reinterpret_cast<u32x4_t*>(smem_raw);
@@ -386,7 +386,7 @@ void k_decode(DecodeArgs a) {
     // this workgroup's slot (the arithmetic below), its expert (the one whose
     // slots hold it), its 16-row chunk and the chunk's tokens, in the sort's
     // order; workgroups past the slots return below
-    const int wps_p = U == ug ? a.wps_guess : slot_wgs<kTwo>(a, U, (int)gridDim.x - 1);
+    const int wps_p = U == ug ? a.wps_guess : slot_wgs<TWO>(a, U, (int)gridDim.x - 1);
     const int slot_p = U == ug ? slot_raw : (int)blockIdx.x / wps_p;
     if (slot_p < U) {
       if (tid < E && pslot[tid] <= slot_p && slot_p < pslot[tid + 1]) psel = tid;
@@ -408,7 +408,7 @@ void k_decode(DecodeArgs a) {
   }
   const bool guessed = U == ug;  // dense: always (u_guess is its slot count)
   const int work_grid = (int)gridDim.x - (SELF != kSelfNone ? 1 : 0);
-  const int wps = guessed ? a.wps_guess : slot_wgs<kTwo>(a, U, work_grid);
+  const int wps = guessed ? a.wps_guess : slot_wgs<TWO>(a, U, work_grid);
   const int slot = guessed ? slot_raw : (int)blockIdx.x / wps;
   const int part = (int)blockIdx.x - slot * wps;
   if (slot >= U) return;  // uniform across the workgroup
@@ -896,7 +896,8 @@ static hipError_t launch_stream(DecodeArgs a, int ncolblk, int max_slots, hipStr
   int64_t grid = std::min<int64_t>(resident, (int64_t)max_slots * a.n_ct);
   if (grid < max_slots) grid = max_slots;
   if (grid <= 0) return hipSuccess;
-  // the slots' second round (slot_wgs): from as many routed rows on as make
+  // the slots' second round (slot_wgs, both kernels alike in registers and
+  // LDS): from as many routed rows on as make
   // it likely.  The workgroups it does not need leave at once, in kSelfPlan
   // after their own plan: 96 tokens x top-8 (128 slots) 108 us with and
   // without them, 96 tokens of skewed routing (145 slots) 144 -> 126 us.
@@ -905,11 +906,14 @@ static hipError_t launch_stream(DecodeArgs a, int ncolblk, int max_slots, hipStr
   // 128 top-4, 256 tokens (G = 128) 142 / 125; 256 and 512 experts, which have
   // more slots than the rule takes, unchanged.
   constexpr int64_t kTwoRoundRows = SELF == kSelfPlan ? 896 : 768;
+  constexpr bool kTwo = two_rounds<MODE, KSPLIT, SELF>();
+  const bool two = kTwo && !narrow && per_cu == 1 && 2 * (int64_t)max_slots > resident &&
+                   (int64_t)a.M * a.topk >= kTwoRoundRows;
   a.resident = 0;
-  if (two_rounds<MODE, KSPLIT, SELF>() && !narrow && per_cu == 1 &&
-      2 * (int64_t)max_slots > resident && (int64_t)a.M * a.topk >= kTwoRoundRows) {
+  if (two) {
     a.resident = (int)resident;
     grid = std::max<int64_t>(grid, std::min<int64_t>(2 * resident, 3 * (int64_t)max_slots));
+    kern = k_decode<MODE, TPW, KSPLIT, LONGK, WIDE, TILED, LSCALE, SELF, kTwo>;
   }
   if (grid >= (1 << 16)) return hipErrorInvalidValue;
   // the kernel's slot arithmetic for max_slots active slots (MoE: the
@@ -917,7 +921,7 @@ static hipError_t launch_stream(DecodeArgs a, int ncolblk, int max_slots, hipStr
   // differs; slot_magic = floor(2^32 / wps) + 1 gives blockIdx.x / wps
   // exactly for blockIdx.x < 2^16
   a.u_guess = std::max(max_slots, 1);
-  a.wps_guess = slot_wgs<two_rounds<MODE, KSPLIT, SELF>()>(a, a.u_guess, (int)grid);
+  a.wps_guess = two ? slot_wgs<true>(a, a.u_guess, (int)grid) : slot_wgs<false>(a, a.u_guess, (int)grid);
   a.slot_magic = a.wps_guess > 1 ? (uint32_t)((1ull << 32) / (uint64_t)a.wps_guess + 1ull) : 0u;
   a.per_guess = (a.n_ct + a.wps_guess - 1) / a.wps_guess;
   // SELF: one more workgroup, the last, writes the plan

@@ -52,13 +52,32 @@ def test_two_rounds_bit_identical(M, n_full, slots, G, tiled):
         assert torch.equal(_lib.moe_forward(x[s], idx[s], wt[s], *ew, G, tiles=tiles), y[s]), f"rows {m}.."
 
 
+# the two-round kernels of the other shapes: two and four k tiles per wavefront, the long-K loop (packed weights only)
+@pytest.mark.parametrize("H,G,tiled", [(1024, 128, False), (1024, 32, False), (1024, 128, True), (1024, 32, True),
+                                       (2048, 128, False), (2048, 32, False), (2048, 128, True), (2048, 32, True),
+                                       (4096, 128, False)])
+def test_two_rounds_other_shapes(H, G, tiled):
+    M, dev = 150, torch.device("cuda:0")
+    w = synth.moe_weights(E, H, I, G, seed=86, device=dev)
+    ew = (w.gate_up_packed, w.gate_up_scale, w.down_packed, w.down_scale)
+    tiles = _lib.tile_experts(*ew, G) if tiled else None
+    idx, n = _routing(M, 20, 82)
+    assert n == 148
+    idx = idx.to(dev)
+    wt = torch.rand(M, K, generator=torch.Generator().manual_seed(83)).to(dev)
+    x = synth.activations(M, H, seed=84, device=dev)
+    y = _lib.moe_forward(x, idx, wt, *ew, G, tiles=tiles)
+    for m in range(0, M, 32):
+        s = slice(m, m + 32)
+        assert torch.equal(_lib.moe_forward(x[s], idx[s], wt[s], *ew, G, tiles=tiles), y[s]), f"rows {m}.."
+
+
 @pytest.mark.parametrize("M,n_full,slots", [(112, 0, 128), (112, 1, 129), (121, 20, 148), (128, 42, 170),
                                             (128, 43, 171)])
-@pytest.mark.parametrize("tiled", [False, True])
-def test_two_rounds_own_plan(M, n_full, slots, tiled):
+@pytest.mark.parametrize("G,tiled", [(128, False), (128, True), (32, True)])
+def test_two_rounds_own_plan(M, n_full, slots, G, tiled):
     # the launch plans for itself (896 <= M * top_k <= 1024); the router's rows make it choose this routing
     dev = torch.device("cuda:0")
-    G = 128
     w = synth.moe_weights(E, H, I, G, seed=91, device=dev)
     ew = (w.gate_up_packed, w.gate_up_scale, w.down_packed, w.down_scale)
     tiles = _lib.tile_experts(*ew, G) if tiled else None
