@@ -27,17 +27,22 @@ __global__ __launch_bounds__(kNormThreads) void k_add_rms_norm(
   const int n8 = H >> 3;
   const uint16_t* hr = h + row * H;
   const uint16_t* dr = delta != nullptr ? delta + row * H : nullptr;
-  u32x4_t xv[NQ], dv[NQ];
+  // every load issued before the first is used, without a branch per chunk
+  // (chunks past the row load its last one again): with one the compiler
+  // waited for a chunk before it asked for the next (rows of 2816 with a
+  // delta, 1 / 4096 of them 2.60 / 13.8 us, so 2.31 / 12.7)
+  u32x4_t xv[NQ], dv[NQ], wv[NQ];
 #pragma unroll
-  for (int q = 0; q < NQ; ++q) {
-    const int c8 = tid + kNormThreads * q;
-    xv[q] = u32x4_t{0u, 0u, 0u, 0u};
-    dv[q] = u32x4_t{0u, 0u, 0u, 0u};
-    if (c8 < n8) {
-      xv[q] = ld16(hr + 8 * c8);
-      if (dr != nullptr) dv[q] = ld16(dr + 8 * c8);
-    }
+  for (int q = 0; q < NQ; ++q) xv[q] = ld16(hr + 8 * min(tid + kNormThreads * q, n8 - 1));
+  if (dr != nullptr) {
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) dv[q] = ld16(dr + 8 * min(tid + kNormThreads * q, n8 - 1));
+  } else {
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) dv[q] = u32x4_t{0u, 0u, 0u, 0u};
   }
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) wv[q] = ld16(w + 8 * min(tid + kNormThreads * q, n8 - 1));
   float ss = 0.f;
 #pragma unroll
   for (int q = 0; q < NQ; ++q) {
@@ -72,9 +77,8 @@ __global__ __launch_bounds__(kNormThreads) void k_add_rms_norm(
   for (int q = 0; q < NQ; ++q) {
     const int c8 = tid + kNormThreads * q;
     if (c8 >= n8) continue;
-    const u32x4_t wv = ld16(w + 8 * c8);
     const uint32_t x4[4] = {xv[q].x, xv[q].y, xv[q].z, xv[q].w};
-    const uint32_t w4[4] = {wv.x, wv.y, wv.z, wv.w};
+    const uint32_t w4[4] = {wv[q].x, wv[q].y, wv[q].z, wv[q].w};
     uint32_t o4[4];
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
