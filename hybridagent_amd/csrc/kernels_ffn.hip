@@ -176,7 +176,9 @@ __global__ __launch_bounds__(kFfnThreads) void k_ffn_post(
   const int n8 = H >> 3;
   Row8 m[NQ], e2[NQ];
   // KMAX > 0: moe holds the expert rows t * topk + j; every slot's index,
-  // weight and chunks are requested before the first is used
+  // weight and chunks are requested before the first is used (slots past topk
+  // load slot 0 again: a branch around a load made the compiler wait for each
+  // chunk's slots before the next's)
   constexpr int KM = KMAX > 0 ? KMAX : 1;
   const int64_t r0 = (int64_t)blockIdx.x * topk;
   int64_t ex[KM];
@@ -193,7 +195,7 @@ __global__ __launch_bounds__(kFfnThreads) void k_ffn_post(
     for (int q = 0; q < NQ; ++q) {
       const int c8 = threadIdx.x + kFfnThreads * q;
 #pragma unroll
-      for (int j = 0; j < KM; ++j) d[q][j] = raw8(moe + (r0 + j) * H, c8, c8 < n8 && j < topk);
+      for (int j = 0; j < KM; ++j) d[q][j] = ld16(moe + (r0 + (j < topk ? j : 0)) * H + 8 * min(c8, n8 - 1));
     }
   }
   // every load issued before the first reduction: the two rows, then the
