@@ -31,7 +31,7 @@ constexpr int kFfnThreads = 256;
 // 16-byte chunks per thread, at most: H <= 256 * 4 * 8.  The kernels are built
 // for NQ = 1 .. 4 of them: with the registers of four a row of 2816 (NQ = 2)
 // kept half the rows in flight (2048 rows: pre 17.8 -> 14.5 us, combine and
-// post 18.3 + 17.7 -> 32.5 us in one launch).
+// post 18.3 + 17.7 -> 30 us in one launch).
 constexpr int kFfnChunks = 4;
 // most slots the combine inside k_ffn_post takes
 constexpr int kFfnTopK = 8;

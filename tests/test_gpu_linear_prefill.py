@@ -39,12 +39,13 @@ def _check(y, x, w, b, K, what):
     assert not bad.any(), f"{what}: {int(bad.sum())} of {bad.numel()}"
 
 
-# the tiled GEMM takes more than 900e3 outputs.  N: one column tile and less, tiles' edges, odd; K: whole and half
-# last stages; rows past whole tiles
+# the tiled GEMM takes more than 900e3 outputs.  N: one column tile and less, tiles' edges, odd; K: whole and partial
+# last tiles; rows past whole tiles; 228 groups (scales fill LDS), 232 and a partial tile past K = 3072 (streamed)
 @pytest.mark.parametrize("M,K,N,G", [(481, 160, 2816, 32), (1001, 160, 2816, 32), (512, 704, 2816, 128),
                                      (700, 2144, 1357, 32), (330, 2816, 2816, 32), (3600, 1056, 257, 64),
                                      (3601, 352, 256, 32), (481, 2080, 2111, 128), (65, 224, 14000, 32),
-                                     (330, 9216, 2816, 128)])
+                                     (330, 9216, 2816, 128), (330, 7296, 2816, 32), (330, 7424, 2816, 32),
+                                     (330, 3232, 2816, 32)])
 def test_linear_prefill_shapes(dev, M, K, N, G):
     p, s, w = _weights(N, K, G, 51, dev)
     x = synth.activations(M, K, 53, dev)
