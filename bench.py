@@ -30,9 +30,9 @@ from HBM.  Times come from HIP events on the stream the kernels run on.
 
 ``roofline`` is the dominant decode kernel (the grouped gate_up GEMM at the
 largest decode M, about two thirds of the decode bytes), timed alone with each
-launch bracketed by its own HIP events (the per-dispatch duration a rocprofv3
-kernel trace of the same command reports; the graph-replay mean is recorded
-beside it); ``roofline_prefill`` the dominant prefill kernel (the gate_up
+launch bracketed by its own HIP events (2 to 4 us above a rocprofv3 kernel
+trace of the same command; the graph-replay mean and the committed trace's are
+recorded beside it); ``roofline_prefill`` the dominant prefill kernel (the gate_up
 stage at M = 4096), timed the same way, against the bf16 MFMA peak, with the
 MFMA-busy fraction of the committed counter summary.  ``g32`` repeats decode (M = 1, 64) and prefill at
 group size 32, the released checkpoints'.
@@ -149,9 +149,9 @@ def time_graph(fn, calls_per_replay: int, steps: int, warmup: int) -> float:
 
 def time_dispatches(fns, reps: int, warmup: int = 1) -> float:
     """Mean seconds per launch with each launch bracketed by its own pair of HIP
-    events on the stream the kernels run on (eager, one after the other): the
-    per-dispatch duration a kernel trace reports, which includes each
-    dispatch's completion and so reads slightly above the graph-replay mean."""
+    events on the stream the kernels run on (eager, one after the other).  It
+    includes each dispatch's completion and so reads above the graph-replay mean
+    and, by 2 to 4 us, above a kernel trace's duration."""
     for _ in range(warmup):
         for f in fns:
             f()
@@ -311,7 +311,7 @@ def roofline_prefill(pre):
         "frac": round(st["tflops"] / PEAK_BF16_TFLOPS, 4),
         "us_per_launch": round(st["us"], 3),
         "us_per_launch_graph_replay": round(st["us_graph"], 3),
-        "timing": "per-dispatch HIP events (each launch bracketed), as a kernel trace reports it",
+        "timing": "per-dispatch HIP events (each launch bracketed)",
         "algorithmic_gflop_per_launch": round(st["gflop"], 3),
         "mfma_busy_frac_counter": counter_summary(PREFILL_COUNTERS_FILE, "mfma_busy_frac_gate_up"),
         "counter_source": os.path.relpath(PREFILL_COUNTERS_FILE, ROOT),
@@ -366,7 +366,7 @@ def roofline(kern):
         "traffic_source": os.path.relpath(TRAFFIC_FILE, ROOT),
         "us_per_launch": round(kern["us"], 3),
         "us_per_launch_graph_replay": round(kern["us_graph"], 3),
-        "timing": "per-dispatch HIP events (each launch bracketed), as a kernel trace reports it",
+        "timing": "per-dispatch HIP events (each launch bracketed)",
         "algorithmic_bytes_per_launch": int(kern["bytes"]),
         # B / us = MB/s: / 1e3 for GB/s
         **trace_fields(ROOF_TRACE_FILE, kern["bytes"], PEAK_HBM_GBS, 1e-3),
